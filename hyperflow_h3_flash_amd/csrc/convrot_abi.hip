@@ -99,6 +99,8 @@ void allow_large_lds() {
                         hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::rotate_lowrank_row_kernel<5>),
                         hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::lowrank_up_rows_kernel<4>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, hf::ur_lds(4));
 #define HF_LR_ATTR(RB, NW)                                                                                \
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::lowrank_down_kernel<RB, NW>),             \
                               hipFuncAttributeMaxDynamicSharedMemorySize, hf::lr_lds(NW));
@@ -668,9 +670,22 @@ bool is_glu(int act_code) { return act_code == HF_ACT_SWIGLU || act_code == HF_A
 // 8 for the 128 x 128 tiles of lowrank_up_kernel, and their stores leave the CU as whole lines behind the next
 // tile's loads. From rank 128: at M=37710 the up projection to N=7168 took 180-220 us on the tiles against 207-270
 // us at rank 256, but 120-140 against 112-120 us at rank 64, where a tile's two stages (one of them zeros) are too
-// short for the persistent pipeline to pay.
+// short for the persistent pipeline to pay. (Where use_up_rows holds too, that kernel runs instead.)
 bool use_up_tiles(int64_t M, int64_t N, int32_t r) {
   return r >= 128 && ((M + hf::GBM - 1) / hf::GBM) * ((N + hf::GBN - 1) / hf::GBN) >= device_cus();
+}
+
+// Whether the up projection keeps u in registers and walks the columns (lowrank_up_rows_kernel): ranks up to 256 (the
+// registers), an output of whole 128-byte lines (its 64-column steps; with ragged lines M=6000, N=7000, r=136 took 64
+// against 55 us on the tiles), and enough (256 rows, 64 columns) steps that loading u and the first slab is a small
+// part of a workgroup's share. Measured against the kernels it replaces there (us): M=37710, N=7168, r=256 186 -> 153,
+// r=192 172 -> 134, r=128 141 -> 124, r=96 159 -> 128, r=64 134 -> 120; N=28672, r=64 466 -> 435; M=41344, N=2048,
+// r=256 66 -> 55; M=8192, N=4096, r=256 (2048 steps) 42 -> 35; equal at 1504 steps (M=12000, N=2048, r=256 23.1) and
+// behind at 768 (M=1536, N=8192, r=192 10.8 -> 12.7), but up to rank 64 ahead from 512 steps on (M=2048, N=4096
+// 8.3 -> 6.9).
+bool use_up_rows(int64_t M, int64_t N, int32_t r) {
+  const int64_t steps = ((M + hf::kUrRows - 1) / hf::kUrRows) * ((N + hf::kUrCols - 1) / hf::kUrCols);
+  return r > 0 && r <= 256 && steps >= (r <= 64 ? 2 : 6) * (int64_t)device_cus();
 }
 
 int64_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, int32_t r, int act_code) {
@@ -953,6 +968,21 @@ int hf_lowrank_up(const uint16_t* u, int64_t ldu, const uint16_t* up, int64_t ld
   if (2 * hf::kUpTile * std::max(ldu, ld_up) >= (int64_t(1) << 31)) return HF_ERR_SIZE;
   allow_large_lds();
   const int vec16 = aligned(y, 16) && (ldy % 8) == 0;
+  if (!bias && aligned(y, 128) && (ldy % 64) == 0 && use_up_rows(M, N, r)) {
+    const int64_t steps_n = (N + hf::kUrCols - 1) / hf::kUrCols;
+    const int64_t steps = ((M + hf::kUrRows - 1) / hf::kUrRows) * steps_n;
+    if (steps >= (int64_t(1) << 31)) return HF_ERR_SIZE;
+    const dim3 grid((unsigned)std::min<int64_t>(2 * device_cus(), steps)), block(hf::kUrThreads);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+#define HF_UR_CASE(RC)                                                                                              \
+  case RC:                                                                                                          \
+    hipLaunchKernelGGL(hf::lowrank_up_rows_kernel<RC>, grid, block, hf::ur_lds(RC), s, u, ldu, up, ld_up, y, ldy,   \
+                       (int)M, (int)N, (int)r, (int)steps_n, (int)steps);                                           \
+    break;
+    switch ((r + 63) / 64) { HF_UR_CASE(1) HF_UR_CASE(2) HF_UR_CASE(3) HF_UR_CASE(4) }
+#undef HF_UR_CASE
+    return launch_status();
+  }
   if (vec16 && use_up_tiles(M, N, r)) {
     // At least a round of 256 x 256 output tiles: the persistent tile kernel's bf16 product (kOutMmBf16), the
     // operands' rows as bytes (2r bytes of rank per row).

@@ -747,4 +747,212 @@ __global__ __launch_bounds__(kUpThreads) void lowrank_up_kernel(const uint16_t* 
   }
 }
 
+// The up projection of many rows at ranks up to 256: the output is written at the rate of the memory. A workgroup of 4
+// waves keeps 256 rows of u in registers (64 rows and every rank to a wave, in the MFMA layout) and walks the columns
+// in steps of 64, the step's up rows going global -> LDS one step ahead into one of two slots. A step's 8 stores per
+// wave are waited for a step later, with the loads issued before them, and two workgroups share a CU, so one computes
+// while the other's stores drain; on the persistent 256 x 256 tiles a tile's stores had to drain before its second K
+// stage, with nothing else on the CU. A workgroup takes an equal share of all (256 rows, 64 columns) steps, columns
+// innermost, so the share may cross from one block of rows to the next. Sums in the order of the other up kernels (K
+// ascending, 16 ranks per MFMA, up as the first operand): the same bits. Bound by the output's stores: M=37710,
+// N=7168 (541 MB written) takes 120-124 us at ranks 64 and 128, 4.4-4.5 TB/s where a plain fill reaches 4.5-4.9; 153
+// us at rank 256 (186 us on the tiles), whose 64 MFMAs per wave and step no longer hide behind them. u loaded in the
+// MFMA layout instead of whole lines cost 7 us at M=5168, N=5376.
+constexpr int kUrRows = 256, kUrCols = 64;
+constexpr int kUrThreads = 256;
+__host__ __device__ constexpr int ur_slot(int rc) { return rc * kUrCols * 128; }             // up rows of a step
+__host__ __device__ constexpr int ur_lds(int rc) { return 2 * ur_slot(rc) + 4 * 32 * 128; }  // + output staging
+
+// RC: 64-rank chunks (r <= 64 RC; ranks past r read as zero).
+template <int RC>
+__global__ __launch_bounds__(kUrThreads, 2) void lowrank_up_rows_kernel(const uint16_t* __restrict__ u, int64_t ldu,
+                                                                        const uint16_t* __restrict__ up, int64_t ldup,
+                                                                        uint16_t* __restrict__ y, int64_t ldy, int M,
+                                                                        int N, int r, int steps_n, int steps) {
+  static_assert(2 * ur_lds(RC) <= 160 * 1024, "two workgroups per CU");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char ur_smem_raw[];
+  unsigned char HF_LDS* smem = (unsigned char HF_LDS*)ur_smem_raw;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sub = lane & 31, half = lane >> 5;
+  unsigned char HF_LDS* staging = smem + 2 * ur_slot(RC) + wave * 4096;
+  const uint32_t ldu_bytes = (uint32_t)ldu * 2u, ldup_bytes = (uint32_t)ldup * 2u;
+  const int first = (int)((int64_t)blockIdx.x * steps / gridDim.x);
+  const int last = (int)((int64_t)(blockIdx.x + 1) * steps / gridDim.x);
+
+  // The up rows of column step j (64 rows of RC 128-byte chunks, each chunk a 64 x 128 byte slab swizzled with
+  // swizzle128) into a slot: 8 RC blocks of 8 rows, 2 RC to a wave. Rows past N and ranks past r read as zero.
+  auto issue = [&](int j, unsigned char HF_LDS* slot) {
+    // An opaque copy of the lane id: keeps the offsets of the loads from staying in registers across the step.
+    int il = lane;
+    asm volatile("" : "+v"(il));
+    const int n0 = j * kUrCols, rows_n = min(kUrCols, N - n0);
+    const uint32_t bytes = (uint32_t)rows_n * ldup_bytes;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(up + (int64_t)n0 * ldup, bytes);
+#pragma unroll
+    for (int i = 0; i < 2 * RC; ++i) {
+      const int blk = wave * 2 * RC + i, row = 8 * (blk & 7) + (il >> 3);
+      const int k = 64 * (blk >> 3) + 8 * swizzle128(row, il & 7);
+      const uint32_t off = ((row < rows_n) & (k < r)) ? (uint32_t)row * ldup_bytes + 2u * (uint32_t)k : bytes;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (void HF_LDS*)(slot + blk * 1024), 16, off, 0, 0, 0);
+    }
+  };
+
+  v8bf uf[4 * RC][2];
+  int mb = first / steps_n, j = first % steps_n, held = -1;
+  if (first < last) issue(j, smem);
+  bool exact = false;  // the previous step issued exactly 8 stores per wave after its loads
+  for (int t = first; t < last; ++t) {
+    unsigned char HF_LDS* slot = smem + ((t - first) & 1) * ur_slot(RC);
+    unsigned char HF_LDS* other = smem + ((t - first + 1) & 1) * ur_slot(RC);
+    const int m0 = mb * kUrRows + wave * 64, n0 = j * kUrCols;
+    // This step's slab has landed (everything issued before the previous step's 8 stores has), and this wave's LDS
+    // reads have returned; the barrier makes both true for every wave, so the other slot can be refilled.
+    if (exact)
+      asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (held != mb) {
+      held = mb;
+      const int rows_m = max(0, min(64, M - m0));
+      const uint32_t bytes = (uint32_t)rows_m * ldu_bytes;
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(u + (int64_t)(rows_m ? m0 : 0) * ldu, bytes);
+      // Whole row segments into the registers (a load in the MFMA layout would touch 32 lines for 32 bytes of each, a
+      // third of the rate), then 32 rows x 64 ranks at a time through the staging area into that layout.
+      int hl = lane;  // opaque, as in issue
+      asm volatile("" : "+v"(hl));
+#pragma unroll
+      for (int c = 0; c < 2 * RC; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int row = 8 * i + (hl >> 3), k = 64 * (c >> 1) + 8 * swizzle128(row, hl & 7);
+          const bool in = (32 * (c & 1) + row < rows_m) & (k < r);
+          const uint32_t off = in ? (uint32_t)(32 * (c & 1) + row) * ldu_bytes + 2u * (uint32_t)k : bytes;
+          uf[4 * (c >> 1) + i][c & 1] = __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+        }
+#pragma unroll
+      for (int c = 0; c < 2 * RC; ++c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *(v8bf HF_LDS*)(staging + i * 1024 + hl * 16) = uf[4 * (c >> 1) + i][c & 1];
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          uf[4 * (c >> 1) + i][c & 1] =
+              *(const v8bf HF_LDS*)(staging + (hl & 31) * 128 + (swizzle128(hl & 31, 2 * i + (hl >> 5)) << 4));
+        wave_lds_sync();
+      }
+    }
+    const int next_j = j + 1 < steps_n ? j + 1 : 0;
+    if (t + 1 < last) issue(next_j, other);
+
+    v16f acc[2][2];
+#pragma unroll
+    for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[ib][b] = (v16f){0};
+    // The up fragments of K step kk + 2 are read while step kk is multiplied, held to that order: left to itself the
+    // compiler reads each fragment right before its two MFMAs and waits for it.
+    v8bf pf[3][2];
+    auto read = [&](int kk) {
+#pragma unroll
+      for (int ib = 0; ib < 2; ++ib) {
+        const int nl = 32 * ib + sub;
+        pf[kk % 3][ib] = *(const v8bf HF_LDS*)(slot + (kk >> 2) * (kUrCols * 128) + nl * 128 +
+                                               (swizzle128(nl, 2 * (kk & 3) + half) << 4));
+      }
+    };
+    read(0);
+    read(1);
+#pragma unroll
+    for (int kk = 0; kk < 4 * RC; ++kk) {
+      if (kk + 2 < 4 * RC) read(kk + 2);
+#pragma unroll
+      for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          acc[ib][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pf[kk % 3][ib], uf[kk][b], acc[ib][b], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // DS read
+#pragma unroll
+    for (int kk = 0; kk < 4 * RC - 2; ++kk) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);  // MFMA
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // bf16 and out through the wave's staging area, 32 rows of 128 bytes at a time: after one exchange between the
+    // lane halves lane (sub, h) holds columns 16h .. 16h + 15 of row sub of each 32 x 32 block, and each store
+    // instruction writes 8 whole 128-byte lines.
+    const bool full = m0 + 64 <= M && n0 + kUrCols <= N;
+    int el = lane;  // opaque, as in issue
+    asm volatile("" : "+v"(el));
+    const int esub = el & 31, ehalf = el >> 5;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int ib = 0; ib < 2; ++ib) {
+        uint32_t w4[4][2];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          w4[g][0] = pack_bf16x2(acc[ib][b][4 * g], acc[ib][b][4 * g + 1]);
+          w4[g][1] = pack_bf16x2(acc[ib][b][4 * g + 2], acc[ib][b][4 * g + 3]);
+        }
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          const auto s02 = __builtin_amdgcn_permlane32_swap(w4[0][w], w4[2][w], false, false);
+          const auto s13 = __builtin_amdgcn_permlane32_swap(w4[1][w], w4[3][w], false, false);
+          w4[0][w] = s02[0];
+          w4[2][w] = s02[1];
+          w4[1][w] = s13[0];
+          w4[3][w] = s13[1];
+        }
+        const int c0 = 4 * ib + 2 * ehalf;
+        *(v4i HF_LDS*)(staging + esub * 128 + (swizzle128(esub, c0) << 4)) =
+            (v4i){(int)w4[0][0], (int)w4[0][1], (int)w4[2][0], (int)w4[2][1]};
+        *(v4i HF_LDS*)(staging + esub * 128 + (swizzle128(esub, c0 + 1) << 4)) =
+            (v4i){(int)w4[1][0], (int)w4[1][1], (int)w4[3][0], (int)w4[3][1]};
+      }
+      wave_lds_sync();
+      v4i val[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 8 * i + (el >> 3);
+        val[i] = *(const v4i HF_LDS*)(staging + row * 128 + (swizzle128(row, el & 7) << 4));
+      }
+      const int n = n0 + 8 * (el & 7);
+      uint16_t* dst = y + (int64_t)(m0 + 32 * b + (el >> 3)) * ldy + n;
+      if (full) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) store_stream(reinterpret_cast<v4i*>(dst + 8 * i * ldy), val[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (m0 + 32 * b + 8 * i + (el >> 3) >= M) continue;
+          if (n + 8 <= N) {
+            *reinterpret_cast<v4i*>(dst + 8 * i * ldy) = val[i];
+          } else {
+            for (int e = 0; e < 8; ++e)
+              if (n + e < N) dst[8 * i * ldy + e] = (uint16_t)((uint32_t)val[i][e >> 1] >> (16 * (e & 1)));
+          }
+        }
+      }
+      wave_lds_sync();  // the next rows rewrite the staging area
+    }
+    exact = full;
+    j = next_j;
+    if (next_j == 0) ++mb;
+  }
+}
+
+template __global__ void lowrank_up_rows_kernel<1>(const uint16_t*, int64_t, const uint16_t*, int64_t, uint16_t*,
+                                                   int64_t, int, int, int, int, int);
+template __global__ void lowrank_up_rows_kernel<2>(const uint16_t*, int64_t, const uint16_t*, int64_t, uint16_t*,
+                                                   int64_t, int, int, int, int, int);
+template __global__ void lowrank_up_rows_kernel<3>(const uint16_t*, int64_t, const uint16_t*, int64_t, uint16_t*,
+                                                   int64_t, int, int, int, int, int);
+template __global__ void lowrank_up_rows_kernel<4>(const uint16_t*, int64_t, const uint16_t*, int64_t, uint16_t*,
+                                                   int64_t, int, int, int, int, int);
+
 }  // namespace hf

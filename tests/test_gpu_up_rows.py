@@ -1,0 +1,72 @@
+"""The low-rank up projection of many rows (u in registers, columns in steps of 64: `lowrank_up_rows_kernel`) against
+the other up kernels on the same inputs, bit for bit (every up kernel adds the ranks in the same order), and sampled
+rows against the oracle's exactly rounded sums.
+
+A zero bias sends the same call to the other kernels: it adds +0 to sums that start from +0, so it changes no bit.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+from golden_utils import within_fp32_sum_bound
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    if not torch.cuda.is_available():
+        pytest.fail("no ROCm device visible")
+    from hyperflow_h3_flash_amd import _native
+
+    _native.library()
+
+
+# Steps of (256 rows, 64 columns), 512 workgroups: a share within one block of rows (N = 28672: 448 steps a block), and
+# shares that cross into the next; ragged last row blocks (one row, less and more than a wave's 64 rows of it); every
+# count of 64-rank chunks, full and with a partial last one; the fewest steps of the route (512 up to rank 64, else 1536).
+@pytest.mark.parametrize("m,n,r", [(2048, 4096, 8), (1793, 4096, 64), (8192, 4096, 72), (6017, 4096, 128),
+                                   (6200, 4096, 136), (24321, 1024, 192), (1000, 28672, 200), (12065, 2112, 256)])
+def test_up_rows_is_bitwise_the_other_kernels(oracle_lib, m, n, r):
+    from hyperflow_h3_flash_amd.int8 import lowrank_up
+
+    steps = -(-m // 256) * -(-n // 64)
+    assert steps >= (512 if r <= 64 else 1536) and n % 64 == 0  # the route at 256 CUs
+    gen = torch.Generator(device=DEV).manual_seed(m + n + r)
+    u = torch.randn(m, r, device=DEV, generator=gen).to(torch.bfloat16)
+    up = (torch.randn(n, r, device=DEV, generator=gen) * 0.1).to(torch.bfloat16)
+    print(f"lowrank_up rows M={m} N={n} r={r}", flush=True)
+    y = lowrank_up(u, up)
+    want = lowrank_up(u, up, torch.zeros(n, device=DEV, dtype=torch.bfloat16))
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+    rows = np.unique(np.concatenate([[0, 63, 64, 255, 256], np.arange(m - 2, m)]))
+    at = torch.from_numpy(rows).to(DEV)
+    bits = lambda t: t.cpu().contiguous().view(torch.int16).numpy().view(np.uint16)  # noqa: E731
+    u_rows, up_bits = bits(u[at]), bits(up)
+    f32 = oracle_lib.bf16_to_f32
+    # an fp32 sum of r products in any order, rounded once
+    assert within_fp32_sum_bound(f32(bits(y[at])), f32(oracle_lib.lowrank_up(u_rows, up_bits)), f32(u_rows),
+                                 f32(up_bits))
+
+
+def test_up_rows_writes_only_its_columns():
+    """A padded output (row stride past N) keeps its padding."""
+    import ctypes
+
+    from hyperflow_h3_flash_amd import _native
+
+    m, n, ld, r = 2100, 4096, 4160, 64
+    u = torch.randn(m, r, device=DEV).to(torch.bfloat16)
+    up = torch.randn(n, r, device=DEV).to(torch.bfloat16)
+    y = torch.full((m, ld), 7.0, device=DEV, dtype=torch.bfloat16)
+    dense = torch.empty(m, n, device=DEV, dtype=torch.bfloat16)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    lib = _native.library()
+    for out, stride in ((y, ld), (dense, n)):
+        assert lib.hf_lowrank_up(u.data_ptr(), r, up.data_ptr(), r, r, None, out.data_ptr(), stride, m, n, stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(y[:, :n], dense) and bool((y[:, n:] == 7.0).all())
