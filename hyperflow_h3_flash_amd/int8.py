@@ -26,7 +26,7 @@ rare one-code roundings, int8.py:23-25; this build always produces the torch-pat
 
 from __future__ import annotations
 
-import ctypes
+import contextlib
 import functools
 from types import SimpleNamespace
 from typing import Any, ClassVar
@@ -187,60 +187,83 @@ class Int8RotLinear(nn.Module):
             cache.update(x=x, version=version, group=self.group, arithmetic=arithmetic, value=quantized)
         return quantized
 
-    def _forward_one_call(self, x: Tensor, x2: Tensor) -> Tensor:
+    def _forward_one_call(self, x: Tensor, x2: Tensor, shape: tuple[int, ...]) -> Tensor:
         """The device layer as one library call (hf_convrot_linear_ws): the same kernels and arithmetic as the
         rotate_quant / lowrank_down / int8_matmul composition, with the host work of a call done once (the shared
-        quantized input of int8.py:150-159 is handled here the same way)."""
-        _check_group(self.group)
-        M, K = x2.shape
-        N = self.out_features
+        quantized input of int8.py:150-159 is handled here the same way). ``x2`` is x as contiguous bf16 rows (x itself
+        when it is that already), ``shape`` the output's leading dimensions.
+
+        With few rows this function, not the GPU, sets the time of a call, so it makes two allocations (the output, and
+        one block for the codes, scales, low-rank intermediate and workspace), reads each parameter once from the
+        module's own dictionaries, and enters a device context only when the input lies on another device than the
+        current one: 27 -> 15 us a call at M=64, K=N=5120, rank 32, whose kernels take 17.5."""
+        group = self.group
+        if group not in DEVICE_GROUPS:
+            _check_group(group)
+        K, N, r = self.in_features, self.out_features, self.rank
+        M = x2.numel() // K
         dev = x2.device
-        act = _activation_code(self.activation)
-        _same_device(dev, self.qweight, self.wscale, self.bias)
+        act = ACTIVATIONS.get(self.activation)
+        if act is None:
+            act = _activation_code(self.activation)
+        w, wscale, bias = _own(self, "qweight"), _own(self, "wscale"), _own(self, "bias")
+        down = up = None
+        if r:
+            down, up = _own(_child(self, "down"), "weight"), _own(_child(self, "up"), "weight")
+        index = x2.get_device()
+        for t in (w, wscale, bias, down, up):
+            if t is not None and t.get_device() != index:
+                _same_device(dev, t)
         cache = Int8RotLinear._last_input
-        version = None if x.is_inference() else x._version
         arithmetic = ARITHMETIC_OPTIONS["rotate_quant"]
-        hit = (cache.get("x") is x and cache.get("version") == version and cache.get("group") == self.group
-               and cache.get("arithmetic") == arithmetic)
+        hit = False
+        if cache or self.keep_input:
+            # Inference tensors (`torch.inference_mode`) have no version counter.
+            version = None if x.is_inference() else x._version
+            hit = (cache.get("x") is x and cache.get("version") == version and cache.get("group") == group
+                   and cache.get("arithmetic") == arithmetic)
+        xq = sx = None
         if hit:
             xq, sx = cache["value"]
-        else:
+        elif self.keep_input:
             xq = torch.empty(M, K, device=dev, dtype=torch.int8)
             sx = torch.empty(M, device=dev, dtype=torch.float32)
-        cache.clear()
+        if cache:
+            cache.clear()
         if self.keep_input:
-            cache.update(x=x, version=version, group=self.group, arithmetic=arithmetic, value=(xq, sx))
-        r = self.rank
-        down = up = u = None
+            cache.update(x=x, version=version, group=group, arithmetic=arithmetic, value=(xq, sx))
         if r:
-            down, up = self.down.weight, self.up.weight
-            _same_device(dev, down, up)
-            if down.dtype != torch.bfloat16 or not down.is_contiguous():
-                down = down.to(torch.bfloat16).contiguous()
-            if up.dtype != torch.bfloat16 or not up.is_contiguous():
-                up = up.to(torch.bfloat16).contiguous()
-            u = torch.empty(M, r, device=dev, dtype=torch.bfloat16)
-        bias = self.bias
-        if bias is not None and (bias.dtype != torch.bfloat16 or not bias.is_contiguous()):
-            bias = bias.to(torch.bfloat16).contiguous()
-        w, ws_ = self.qweight, self.wscale
+            down, up = _bf16(down), _bf16(up)
+        if bias is not None:
+            bias = _bf16(bias)
         if not w.is_contiguous():
             w = w.contiguous()
-        if ws_.dtype != torch.float32 or not ws_.is_contiguous():
-            ws_ = ws_.to(torch.float32).contiguous()
-        y = torch.empty(M, N // 2 if act in _GLU_CODES else N, device=dev, dtype=torch.bfloat16)
+        if wscale.dtype is not torch.float32 or not wscale.is_contiguous():
+            wscale = wscale.to(torch.float32).contiguous()
+        n_out = N // 2 if act in _GLU_CODES else N
+        y = torch.empty((*shape, n_out), device=dev, dtype=torch.bfloat16)
         lib = _native.library()
         key = (M, N, K, r, act)
         nbytes = _ONE_CALL_WS.get(key)
         if nbytes is None:
-            nbytes = _ONE_CALL_WS[key] = lib.hf_convrot_linear_ws_bytes(M, N, K, r, act)
-        with torch.cuda.device(dev):
-            work = torch.empty(nbytes, device=dev, dtype=torch.uint8) if nbytes > 0 else None
-            status = lib.hf_convrot_linear_ws(
-                _ptr(x2), x2.stride(0), _ptr(xq), _ptr(sx), int(hit), ROTATE_ARITHMETICS[arithmetic],
-                _ptr(w), w.stride(0), _ptr(ws_), _ptr(down), down.stride(0) if r else 0, _ptr(up),
-                up.stride(0) if r else 0, r, _ptr(bias), act, self.group, _ptr(u), _ptr(y), y.stride(0), M, N, K,
-                _ptr(work), nbytes if work is not None else 0, _stream(dev))
+            nbytes = _ONE_CALL_WS[key] = max(lib.hf_convrot_linear_ws_bytes(M, N, K, r, act), 0)
+        # One block, its parts on 256-byte boundaries: codes and scales (unless they are shared), u, workspace.
+        at_sx = at_u = 0
+        if xq is None:
+            at_sx = _up256(M * K)
+            at_u = at_sx + _up256(4 * M)
+        at_ws = at_u + _up256(2 * M * r)
+        size = at_ws + nbytes
+        scratch = torch.empty(size, device=dev, dtype=torch.uint8) if size else None
+        base = scratch.data_ptr() if size else 0
+        args = (
+            x2.data_ptr(), K, base if xq is None else xq.data_ptr(), base + at_sx if xq is None else sx.data_ptr(),
+            hit, ROTATE_ARITHMETICS[arithmetic], w.data_ptr(), w.stride(0), wscale.data_ptr(),
+            down.data_ptr() if r else None, down.stride(0) if r else 0, up.data_ptr() if r else None,
+            up.stride(0) if r else 0, r, None if bias is None else bias.data_ptr(), act, group,
+            base + at_u if r else None, y.data_ptr(), n_out, M, N, K, base + at_ws if nbytes else None, nbytes)
+        with _on(dev):
+            status = lib.hf_convrot_linear_ws(*args, _raw_stream(index))
         _check(status, "hf_convrot_linear_ws")
         return y
 
@@ -257,11 +280,15 @@ class Int8RotLinear(nn.Module):
 
     def forward(self, x: Tensor) -> Tensor:
         shape = x.shape
-        x2 = x.reshape(-1, self.in_features).to(torch.bfloat16).contiguous()
+        if (x.dtype is torch.bfloat16 and shape and shape[-1] == self.in_features and x.is_contiguous()
+                and x.numel()):
+            x2 = x  # rows of bf16 already: every kernel call below takes it as it is
+        else:
+            x2 = x.reshape(-1, self.in_features).to(torch.bfloat16).contiguous()
         if not x2.is_cuda:
             # Host tensors: the same arithmetic on the CPU (the reference's torch branch, int8.py:164-167).
             Int8RotLinear._last_input.clear()
-            y = self._forward_torch(x2)
+            y = self._forward_torch(x2.reshape(-1, self.in_features))
             return y.reshape(*shape[:-1], y.shape[-1]).to(x.dtype)
         kernels = _kernels()
         if kernels is None:
@@ -272,8 +299,11 @@ class Int8RotLinear(nn.Module):
             )
         if (kernels.rotate_quant is rotate_quant and kernels.lowrank_down is lowrank_down
                 and kernels.int8_matmul is int8_matmul and self.rank % 8 == 0):
-            y = self._forward_one_call(x, x2)
+            if x2 is x:
+                return self._forward_one_call(x, x2, shape[:-1])
+            y = self._forward_one_call(x, x2, (x2.shape[0],))
             return y.reshape(*shape[:-1], y.shape[-1]).to(x.dtype)
+        x2 = x2.reshape(-1, self.in_features)
         xq, sx = self._quantize(x, x2, kernels)
         if self.rank:
             u = kernels.lowrank_down(x2, self.down.weight)
@@ -291,8 +321,25 @@ def _ptr(t: Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _up256(nbytes: int) -> int:
+    return (nbytes + 255) & ~255
+
+
+def _own(module: nn.Module, name: str) -> Tensor | None:
+    """``getattr(module, name)`` for a parameter, from the module's own dictionary when it is there (nn.Module finds
+    its parameters only after the ordinary lookup has failed)."""
+    p = module._parameters.get(name)
+    return getattr(module, name) if p is None else p
+
+
+def _child(module: nn.Module, name: str) -> nn.Module:
+    m = module._modules.get(name)
+    return getattr(module, name) if m is None else m
+
+
+#: The current stream's handle of a device index, without building a Stream object.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def _workspace(device: torch.device, nbytes: int) -> tuple[Tensor | None, int]:
@@ -300,6 +347,20 @@ def _workspace(device: torch.device, nbytes: int) -> tuple[Tensor | None, int]:
     if nbytes <= 0:
         return None, 0
     return torch.empty(nbytes, device=device, dtype=torch.uint8), nbytes
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """A context in which ``device`` is current: nothing to do when it is already."""
+    here = device.index is not None and torch.cuda.current_device() == device.index
+    return _HERE if here else torch.cuda.device(device)
+
+
+def _bf16(t: Tensor) -> Tensor:
+    """``t.to(torch.bfloat16).contiguous()``, without the two calls when it is that already."""
+    return t if t.dtype is torch.bfloat16 and t.is_contiguous() else t.to(torch.bfloat16).contiguous()
 
 
 def _check(status: int, what: str) -> None:
@@ -331,9 +392,10 @@ def rotate_quant(x: Tensor, group: int, arithmetic: str | None = None) -> tuple[
     M, K = x.shape
     q = torch.empty(M, K, device=x.device, dtype=torch.int8)
     s = torch.empty(M, device=x.device, dtype=torch.float32)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         status = _native.library().hf_rotate_quant_ex(_ptr(x), x.stride(0), _ptr(q), q.stride(0), _ptr(s), M, K,
-                                                      group, ROTATE_ARITHMETICS[arithmetic], _stream(x.device))
+                                                      group, ROTATE_ARITHMETICS[arithmetic],
+                                                      _raw_stream(x.device.index))
     _check(status, "hf_rotate_quant_ex")
     return q, s
 
@@ -343,13 +405,13 @@ def lowrank_down(x: Tensor, down: Tensor) -> Tensor:
     M, K = x.shape
     r = down.shape[0]
     _same_device(x.device, down)
-    down = down.to(torch.bfloat16).contiguous()
+    down = _bf16(down)
     u = torch.empty(M, r, device=x.device, dtype=torch.bfloat16)
     lib = _native.library()
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         ws, nbytes = _workspace(x.device, lib.hf_lowrank_down_ws_bytes(M, K, r))
         status = lib.hf_lowrank_down_ws(_ptr(x), x.stride(0), _ptr(down), down.stride(0), _ptr(u), u.stride(0), M, K,
-                                        r, _ptr(ws), nbytes, _stream(x.device))
+                                        r, _ptr(ws), nbytes, _raw_stream(x.device.index))
     _check(status, "hf_lowrank_down_ws")
     return u
 
@@ -361,13 +423,14 @@ def lowrank_up(u: Tensor, up: Tensor, bias: Tensor | None = None) -> Tensor:
     if up.shape[1] != r:
         raise ValueError(f"rank mismatch: {tuple(u.shape)} vs {tuple(up.shape)}")
     _same_device(u.device, up, bias)
-    u, up = _pad_rank(u.to(torch.bfloat16), up.to(torch.bfloat16))
+    u, up = _pad_rank(_bf16(u), _bf16(up))
     if bias is not None:
-        bias = bias.to(torch.bfloat16).contiguous()
+        bias = _bf16(bias)
     y = torch.empty(M, N, device=u.device, dtype=torch.bfloat16)
-    with torch.cuda.device(u.device):
+    with _on(u.device):
         status = _native.library().hf_lowrank_up(_ptr(u), u.stride(0), _ptr(up), up.stride(0), u.shape[1],
-                                                 _ptr(bias), _ptr(y), y.stride(0), M, N, _stream(u.device))
+                                                 _ptr(bias), _ptr(y), y.stride(0), M, N,
+                                                 _raw_stream(u.device.index))
     _check(status, "hf_lowrank_up")
     return y
 
@@ -377,8 +440,7 @@ def _pad_rank(u: Tensor, up: Tensor) -> tuple[Tensor, Tensor]:
     r = u.shape[1]
     pad = -r % 8
     if pad:
-        u = torch.nn.functional.pad(u, (0, pad))
-        up = torch.nn.functional.pad(up, (0, pad))
+        return torch.nn.functional.pad(u, (0, pad)).contiguous(), torch.nn.functional.pad(up, (0, pad)).contiguous()
     return u.contiguous(), up.contiguous()
 
 
@@ -423,12 +485,12 @@ def int8_matmul(a: Tensor, b: Tensor, sa: Tensor, sb: Tensor, *, u: Tensor | Non
         bias = bias.to(torch.bfloat16).contiguous()
     c = torch.empty(M, N // 2 if act in _GLU_CODES else N, device=a.device, dtype=torch.bfloat16)
     lib = _native.library()
-    with torch.cuda.device(a.device):
+    with _on(a.device):
         ws, nbytes = _workspace(a.device, lib.hf_int8_linear_ws_bytes(M, N, K, r, act))
         status = lib.hf_int8_linear_act_ws(
             _ptr(a), a.stride(0), _ptr(b), b.stride(0), _ptr(sa), _ptr(sb),
             _ptr(u), u.stride(0) if u is not None else 0, _ptr(up), up.stride(0) if up is not None else 0, r,
-            _ptr(bias), act, _ptr(c), c.stride(0), M, N, K, _ptr(ws), nbytes, _stream(a.device))
+            _ptr(bias), act, _ptr(c), c.stride(0), M, N, K, _ptr(ws), nbytes, _raw_stream(a.device.index))
     _check(status, "hf_int8_linear_act_ws")
     return c
 
@@ -440,9 +502,9 @@ def int8_gemm_i32(a: Tensor, b: Tensor) -> Tensor:
     _same_device(a.device, b)
     a, b = a.contiguous(), b.contiguous()
     acc = torch.empty(M, N, device=a.device, dtype=torch.int32)
-    with torch.cuda.device(a.device):
+    with _on(a.device):
         status = _native.library().hf_int8_gemm_i32(_ptr(a), a.stride(0), _ptr(b), b.stride(0), _ptr(acc),
-                                                    acc.stride(0), M, N, K, _stream(a.device))
+                                                    acc.stride(0), M, N, K, _raw_stream(a.device.index))
     _check(status, "hf_int8_gemm_i32")
     return acc
 
