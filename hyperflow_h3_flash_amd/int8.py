@@ -27,6 +27,7 @@ rare one-code roundings, int8.py:23-25; this build always produces the torch-pat
 from __future__ import annotations
 
 import contextlib
+import ctypes
 import functools
 from types import SimpleNamespace
 from typing import Any, ClassVar
@@ -337,6 +338,10 @@ def _child(module: nn.Module, name: str) -> nn.Module:
     return getattr(module, name) if m is None else m
 
 
+def _stream(device: torch.device) -> ctypes.c_void_p:
+    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
 #: The current stream's handle of a device index, without building a Stream object.
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
     lambda index: torch.cuda.current_stream(index).cuda_stream)
@@ -490,7 +495,7 @@ def int8_matmul(a: Tensor, b: Tensor, sa: Tensor, sb: Tensor, *, u: Tensor | Non
         status = lib.hf_int8_linear_act_ws(
             _ptr(a), a.stride(0), _ptr(b), b.stride(0), _ptr(sa), _ptr(sb),
             _ptr(u), u.stride(0) if u is not None else 0, _ptr(up), up.stride(0) if up is not None else 0, r,
-            _ptr(bias), act, _ptr(c), c.stride(0), M, N, K, _ptr(ws), nbytes, _raw_stream(a.device.index))
+            _ptr(bias), act, _ptr(c), c.stride(0), M, N, K, _ptr(ws), nbytes, _stream(a.device))
     _check(status, "hf_int8_linear_act_ws")
     return c
 
@@ -504,7 +509,7 @@ def int8_gemm_i32(a: Tensor, b: Tensor) -> Tensor:
     acc = torch.empty(M, N, device=a.device, dtype=torch.int32)
     with _on(a.device):
         status = _native.library().hf_int8_gemm_i32(_ptr(a), a.stride(0), _ptr(b), b.stride(0), _ptr(acc),
-                                                    acc.stride(0), M, N, K, _raw_stream(a.device.index))
+                                                    acc.stride(0), M, N, K, _stream(a.device))
     _check(status, "hf_int8_gemm_i32")
     return acc
 
