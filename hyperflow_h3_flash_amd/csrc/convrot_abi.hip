@@ -102,8 +102,12 @@ void allow_large_lds() {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::lowrank_up_rows_kernel<4>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, hf::ur_lds(4));
 #define HF_LR_ATTR(RB, NW)                                                                                \
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::lowrank_down_kernel<RB, NW>),             \
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::lowrank_down_kernel<RB, NW, hf::kCpolStream>), \
                               hipFuncAttributeMaxDynamicSharedMemorySize, hf::lr_lds(NW));
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::lowrank_down_kernel<1, 4, 0>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, hf::lr_lds(4));
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::lowrank_down_kernel<2, 4, 0>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, hf::lr_lds(4));
     HF_LR_ATTR(1, 4) HF_LR_ATTR(1, 5) HF_LR_ATTR(1, 6) HF_LR_ATTR(1, 7) HF_LR_ATTR(1, 8)
     HF_LR_ATTR(2, 4) HF_LR_ATTR(2, 5) HF_LR_ATTR(2, 6) HF_LR_ATTR(2, 7) HF_LR_ATTR(2, 8)
 #undef HF_LR_ATTR
@@ -413,6 +417,12 @@ int lowrank_down_impl(const uint16_t* x, int64_t ldx, const uint16_t* down, int6
     return HF_OK;
   }
   float* part = plan.splits > 1 ? static_cast<float*>(ws) : nullptr;
+  // A split projection runs before the layer's rotation, which reads x again. x that fits the eight XCDs' L2s (4 MiB
+  // each) is left there for it; a larger x is streamed past the caches: the rotation of that many rows is bound by its
+  // arithmetic, and x would push the codes and weights out. Layers, cached against streamed (same box, in turn): M=1000,
+  // K=5120 (10 MB) 50.1 against 50.7 us, M=1024, K=3072 30.2 against 31.0; M=5168, K=5120 (53 MB) 170.4 against 166.1,
+  // M=5168 feed-forward (53 and 143 MB) 813 against 811.
+  const bool cache_x = part && 2 * M * K <= (int64_t(32) << 20);
   // Waves per workgroup (32 rows each): the fewest that cover the rows in one round of one workgroup per CU, from 4
   // (128 rows) to 8; split launches keep 4.
   int nw = 4;
@@ -426,16 +436,18 @@ int lowrank_down_impl(const uint16_t* x, int64_t ldx, const uint16_t* down, int6
     const uint16_t* d = down + (int64_t)j0 * ld_down;
     uint16_t* uo = u + j0;
     const dim3 grid(blocks, (unsigned)plan.splits), block(64 * nw);
+#define HF_LR_LAUNCH(RB, NW, CPOL)                                                                                  \
+  hipLaunchKernelGGL((hf::lowrank_down_kernel<RB, NW, CPOL>), grid, block, hf::lr_lds(NW), s, x, ldx, d, ld_down,   \
+                     uo, ldu, (int)M, (int)K, rr, plan.k_chunk, part)
 #define HF_LR_CASE(NW)                                                                                              \
-  if (nw == NW) {                                                                                                   \
-    if (rr <= 32)                                                                                                   \
-      hipLaunchKernelGGL((hf::lowrank_down_kernel<1, NW>), grid, block, hf::lr_lds(NW), s, x, ldx, d, ld_down, uo,  \
-                         ldu, (int)M, (int)K, rr, plan.k_chunk, part);                                              \
-    else                                                                                                            \
-      hipLaunchKernelGGL((hf::lowrank_down_kernel<2, NW>), grid, block, hf::lr_lds(NW), s, x, ldx, d, ld_down, uo,  \
-                         ldu, (int)M, (int)K, rr, plan.k_chunk, part);                                              \
+  else if (nw == NW) {                                                                                              \
+    if (rr <= 32) HF_LR_LAUNCH(1, NW, hf::kCpolStream); else HF_LR_LAUNCH(2, NW, hf::kCpolStream);                   \
   }
+    if (cache_x) {
+      if (rr <= 32) HF_LR_LAUNCH(1, 4, 0); else HF_LR_LAUNCH(2, 4, 0);
+    }
     HF_LR_CASE(4) HF_LR_CASE(5) HF_LR_CASE(6) HF_LR_CASE(7) HF_LR_CASE(8)
+#undef HF_LR_LAUNCH
 #undef HF_LR_CASE
     int st = launch_status();
     if (st != HF_OK) return st;
