@@ -125,6 +125,10 @@ void allow_large_lds() {
                               hipFuncAttributeMaxDynamicSharedMemorySize, hf::kMidLds);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::mid_gemm_kernel<hf::kActGeluTanh>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, hf::kMidLds);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::mid_gemm_kernel<hf::kActNone, hf::kMidStreamW>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, hf::kMidLds);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::mid_gemm_kernel<hf::kActGeluTanh, hf::kMidStreamW>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, hf::kMidLds);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&hf::lowrank_down_band_kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, hf::kLbLds);
 #define HF_BAND_ATTR(NB)                                                                                            \
@@ -773,10 +777,20 @@ int int8_linear_impl(const int8_t* q, int64_t ldq, const int8_t* w, int64_t ldw,
     a.tiles_n = (int)((N + hf::kMidBN - 1) / hf::kMidBN);
     a.out_vec16 = aligned(y, 16) && (ldy % 8) == 0;
     const dim3 grid((unsigned)((int64_t)a.tiles_m * a.tiles_n)), block(hf::kMidThreads);
-    if (act == hf::kActGeluTanh)
-      hipLaunchKernelGGL(hf::mid_gemm_kernel<hf::kActGeluTanh>, grid, block, hf::kMidLds, s, a);
-    else
-      hipLaunchKernelGGL(hf::mid_gemm_kernel<hf::kActNone>, grid, block, hf::kMidLds, s, a);
+    // One row of tiles (M <= 256) reads every weight panel once: a weight of more than half the 256 MiB Infinity Cache
+    // is streamed, so it leaves the codes in the L2s and does not sweep that cache for nothing. Layers, both orders on
+    // one box: M=256, N=30720, K=5120 (157 MB) 64.9 -> 62.8 us, M=200 62.0 -> 59.9, M=130, N=28672, K=5376 54.9 -> 54.0,
+    // K=7168 (220 MB) 79.5 -> 78.6. Smaller weights may still be there from the call before (M=256, N=22016, K=3072, 68
+    // MB, called over three weights 35.9 -> 39.1), and with more tile rows the panels are read again (M=1024, N=7168,
+    // K=5120 57.9 -> 59.8).
+    const bool stream_w = a.tiles_m == 1 && N * K > (int64_t(128) << 20);
+#define HF_MID_LAUNCH(ACT)                                                                                          \
+    if (stream_w)                                                                                                   \
+      hipLaunchKernelGGL((hf::mid_gemm_kernel<ACT, hf::kMidStreamW>), grid, block, hf::kMidLds, s, a);              \
+    else                                                                                                            \
+      hipLaunchKernelGGL((hf::mid_gemm_kernel<ACT, 0>), grid, block, hf::kMidLds, s, a);
+    if (act == hf::kActGeluTanh) { HF_MID_LAUNCH(hf::kActGeluTanh) } else { HF_MID_LAUNCH(hf::kActNone) }
+#undef HF_MID_LAUNCH
     return launch_status();
   }
   if (route.kind == GemmRoute::kSkinnyFused) {

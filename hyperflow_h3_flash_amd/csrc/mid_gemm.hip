@@ -70,7 +70,10 @@ __device__ __forceinline__ void mid_tile_of(int bid, int tiles_m, int tiles_n, i
   tn = logical / tiles_m;
 }
 
-template <int ACT>
+// WPOL: the cache policy of the weight's loads, kMidStreamW (the non-temporal hint) where one row of tiles reads every
+// weight panel once (the host's choice).
+constexpr int kMidStreamW = 2;
+template <int ACT, int WPOL = 0>
 __global__ __launch_bounds__(kMidThreads, 1) void mid_gemm_kernel(MidArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char mid_smem_raw[];
   unsigned char HF_LDS* smem = (unsigned char HF_LDS*)mid_smem_raw;
@@ -128,8 +131,11 @@ __global__ __launch_bounds__(kMidThreads, 1) void mid_gemm_kernel(MidArgs a) {
       const uint32_t col = (uint32_t)col0 + chunk;
       const uint32_t voff = ((row < rows) & (col < (uint32_t)limit)) ? (uint32_t)(row * (isb ? ld_b : ld_a)) + col
                                                                        : (isb ? oob_b : oob_a);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(isb ? rb : ra, (void HF_LDS*)(dst + (isb ? kMidAStage : 0) + blk * 1024),
-                                               16, voff, 0, 0, 0);
+      unsigned char HF_LDS* to = dst + (isb ? kMidAStage : 0) + blk * 1024;
+      if (isb)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (void HF_LDS*)to, 16, voff, 0, 0, WPOL);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (void HF_LDS*)to, 16, voff, 0, 0, 0);
     }
   };
 
@@ -329,6 +335,8 @@ __global__ __launch_bounds__(kMidThreads, 1) void mid_gemm_kernel(MidArgs a) {
 
 template __global__ void mid_gemm_kernel<kActNone>(MidArgs);
 template __global__ void mid_gemm_kernel<kActGeluTanh>(MidArgs);
+template __global__ void mid_gemm_kernel<kActNone, kMidStreamW>(MidArgs);
+template __global__ void mid_gemm_kernel<kActGeluTanh, kMidStreamW>(MidArgs);
 
 // ------------------------------------------------------------------------------------------------- 128-row bands
 // band_gemm_kernel<NB>: 128 (m) x 32 NB (n) output tiles, one per workgroup, for shapes whose 256 x 128 tiles leave
