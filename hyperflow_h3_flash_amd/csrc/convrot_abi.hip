@@ -701,7 +701,7 @@ bool use_up_tiles(int64_t M, int64_t N, int32_t r) {
 // 8.3 -> 6.9).
 bool use_up_rows(int64_t M, int64_t N, int32_t r) {
   const int64_t steps = ((M + hf::kUrRows - 1) / hf::kUrRows) * ((N + hf::kUrCols - 1) / hf::kUrCols);
-  return r > 0 && r <= 256 && steps >= (r <= 64 ? 2 : 6) * (int64_t)device_cus();
+  return r > 0 && r <= 256 && steps >= (r <= 64 ? 2 : 6) * (int64_t)device_cus() && steps < (int64_t(1) << 31);
 }
 
 int64_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, int32_t r, int act_code) {
@@ -997,7 +997,6 @@ int hf_lowrank_up(const uint16_t* u, int64_t ldu, const uint16_t* up, int64_t ld
   if (!bias && aligned(y, 128) && (ldy % 64) == 0 && use_up_rows(M, N, r)) {
     const int64_t steps_n = (N + hf::kUrCols - 1) / hf::kUrCols;
     const int64_t steps = ((M + hf::kUrRows - 1) / hf::kUrRows) * steps_n;
-    if (steps >= (int64_t(1) << 31)) return HF_ERR_SIZE;
     const dim3 grid((unsigned)std::min<int64_t>(2 * device_cus(), steps)), block(hf::kUrThreads);
     hipStream_t s = static_cast<hipStream_t>(stream);
 #define HF_UR_CASE(RC)                                                                                              \
