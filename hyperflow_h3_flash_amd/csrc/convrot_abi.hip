@@ -1102,13 +1102,21 @@ namespace {
 
 // The rotation (bf16_div arithmetic) and the low-rank down projection of a few rows in one launch
 // (rotate_lowrank_row_kernel): the argument rules of hf_rotate_quant and hf_lowrank_down together. Used when both
-// would run their row kernels and the rows are few: the low-rank workgroups take the rotation's dynamic LDS (about
-// 11 KiB per 1024-element tile), so with more rows they fit fewer per CU than alone. Layer A/B (HIP graph, N=5120,
-// rank 64): one launch ahead by 1-5 us up to 128 rows at every K and up to 192 rows at 7 or fewer tiles; behind by
-// 1-8 us at 256-384 rows with K=5120 or K=14336.
-bool rotate_lowrank_by_rows(int64_t M, int64_t K) {
+// would run their row kernels and the launch's workgroups are few: the low-rank ones take the rotation's dynamic LDS
+// (about 11 KiB per 1024-element tile), so fewer fit per CU than alone. Layer A/B (HIP graph, N=5120, rank 64): one
+// launch ahead by 1-5 us up to 128 rows at every K and up to 192 rows at 7 or fewer tiles; behind by 1-8 us at 256-384
+// rows with K=5120 or K=14336. Past those rows it is the workgroups that count, in rounds of what the CUs hold at once
+// (N=5120, us a layer, apart / one launch): up to 5 tiles ahead to 3.4 rounds (M=256, K=3072, rank 32 27.9 / 25.7;
+// M=384, rank 64 37.2 / 35.0; M=300, K=5120, rank 32 39.7 / 38.0) and equal at 4.5 (M=256, K=5120, rank 64 37.5 / 37.6),
+// with more tiles ahead to 2 (M=200, K=7168, rank 32 35.1 / 32.1) and behind at 2.5 and more (M=256 34.5 / 35.4; M=160,
+// K=10240 37.3 / 38.2). That rule applies where the projection alone would run by rows too, so the sums are the same.
+bool rotate_lowrank_by_rows(int64_t M, int64_t K, int32_t r) {
   const int64_t ntiles = (K + hf::kRqTile - 1) / hf::kRqTile;
-  return lowrank_by_rows(M, K) && M <= kRowKernelMaxRows && ntiles <= 14 && (M <= 128 || (M <= 192 && ntiles <= 7));
+  if (!lowrank_by_rows(M, K) || M > kRowKernelMaxRows || ntiles > 14) return false;
+  if (M <= 128 || (M <= 192 && ntiles <= 7)) return true;
+  const int64_t per_cu = kMaxLds / (int64_t)hf::rotate_quant_row_lds_bytes((int)K);
+  const int64_t wgs = hf::lowrank_row_blocks(M, r) + M;
+  return lowrank_rows_faster(M, K) && 2 * wgs <= (ntiles <= 5 ? 7 : 4) * per_cu * device_cus();
 }
 
 int rotate_lowrank_rows(const uint16_t* x, int64_t ldx, int8_t* q, int64_t ldq, float* sx, const uint16_t* down,
@@ -1161,7 +1169,7 @@ int hf_convrot_linear_ws(const uint16_t* x, int64_t ldx, int8_t* q, float* sx, i
   if (M < 0 || N < 0 || K <= 0 || r < 0) return HF_ERR_ARGUMENT;
   if (M == 0 || N == 0) return HF_OK;
   int st = HF_OK;
-  if (!quantized && r > 0 && arithmetic == HF_ROTATE_BF16_DIV && group <= 1024 && rotate_lowrank_by_rows(M, K)) {
+  if (!quantized && r > 0 && arithmetic == HF_ROTATE_BF16_DIV && group <= 1024 && rotate_lowrank_by_rows(M, K, r)) {
     st = rotate_lowrank_rows(x, ldx, q, K, sx, down, ld_down, u, r, M, K, r, group, stream);
     if (st != HF_OK) return st;
   } else if (!quantized && r > 0 && arithmetic == HF_ROTATE_BF16_DIV && lowrank_split_planned(M, K, r, ws, ws_bytes)) {
