@@ -180,9 +180,10 @@ class Int8RotLinear(nn.Module):
         # Inference tensors (`torch.inference_mode`) have no version counter.
         version = None if x.is_inference() else x._version
         arithmetic = ARITHMETIC_OPTIONS["rotate_quant"]
-        hit = (cache.get("x") is x and cache.get("version") == version and cache.get("group") == self.group
-               and cache.get("arithmetic") == arithmetic)
-        quantized = cache["value"] if hit else kernels.rotate_quant(x2, self.group)
+        entry = dict(cache)  # one copy: another thread may drop or replace the entry between the checks
+        hit = (entry.get("x") is x and entry.get("version") == version and entry.get("group") == self.group
+               and entry.get("arithmetic") == arithmetic)
+        quantized = entry["value"] if hit else kernels.rotate_quant(x2, self.group)
         cache.clear()
         if self.keep_input:
             cache.update(x=x, version=version, group=self.group, arithmetic=arithmetic, value=quantized)
@@ -217,22 +218,22 @@ class Int8RotLinear(nn.Module):
                 _same_device(dev, t)
         cache = Int8RotLinear._last_input
         arithmetic = ARITHMETIC_OPTIONS["rotate_quant"]
-        hit = False
-        if cache or self.keep_input:
-            # Inference tensors (`torch.inference_mode`) have no version counter.
-            version = None if x.is_inference() else x._version
-            hit = (cache.get("x") is x and cache.get("version") == version and cache.get("group") == group
-                   and cache.get("arithmetic") == arithmetic)
+        keep, hit = self.keep_input, False
         xq = sx = None
-        if hit:
-            xq, sx = cache["value"]
-        elif self.keep_input:
+        if cache or keep:
+            # Inference tensors (`torch.inference_mode`) have no version counter. One copy of the entry: another thread
+            # may drop or replace it between the checks.
+            entry = dict(cache)
+            version = None if x.is_inference() else x._version
+            hit = (entry.get("x") is x and entry.get("version") == version and entry.get("group") == group
+                   and entry.get("arithmetic") == arithmetic)
+            if hit:
+                xq, sx = entry["value"]
+            del entry
+            cache.clear()
+        if keep and not hit:
             xq = torch.empty(M, K, device=dev, dtype=torch.int8)
             sx = torch.empty(M, device=dev, dtype=torch.float32)
-        if cache:
-            cache.clear()
-        if self.keep_input:
-            cache.update(x=x, version=version, group=group, arithmetic=arithmetic, value=(xq, sx))
         if r:
             down, up = _bf16(down), _bf16(up)
         if bias is not None:
@@ -266,6 +267,9 @@ class Int8RotLinear(nn.Module):
         with _on(dev):
             status = lib.hf_convrot_linear_ws(*args, _raw_stream(index))
         _check(status, "hf_convrot_linear_ws")
+        # Left behind only now: before the call xq and sx hold nothing, and a call that fails leaves nothing to share.
+        if keep:
+            cache.update(x=x, version=version, group=group, arithmetic=arithmetic, value=(xq, sx))
         return y
 
     def _forward_torch(self, x2: Tensor, rot: Tensor | None = None) -> Tensor:

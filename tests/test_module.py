@@ -3,6 +3,7 @@
 
 from __future__ import annotations
 
+import contextlib
 import io
 from types import SimpleNamespace
 
@@ -174,6 +175,64 @@ def test_shared_quantization_invalidated_by_in_place_change_and_other_tensors():
     to_other._quantize(x, x, kernels)  # same tensor, other group
     assert len(calls) == 4
     Int8RotLinear._last_input.clear()
+
+
+class _StubLibrary:
+    """The one-call entry point without a device: records its `quantized` argument and returns `status`."""
+
+    def __init__(self):
+        self.quantized, self.status = [], 0
+
+    def hf_convrot_linear_ws_bytes(self, *sizes):
+        return 0
+
+    def hf_convrot_linear_ws(self, *args):
+        self.quantized.append(bool(args[4]))
+        return self.status
+
+    def hf_strerror(self, status):
+        return b"stub"
+
+
+@pytest.fixture
+def stub_library(monkeypatch):
+    lib = _StubLibrary()
+    monkeypatch.setattr(int8_mod._native, "library", lambda: lib)
+    monkeypatch.setattr(int8_mod, "_on", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(int8_mod, "_raw_stream", lambda index: 0)
+    Int8RotLinear._last_input.clear()
+    yield lib
+    Int8RotLinear._last_input.clear()
+
+
+@pytest.mark.parametrize("fails", ["status", "output allocation"])
+def test_a_failed_layer_leaves_no_codes_to_share(stub_library, monkeypatch, fails):
+    """The codes are shared only once the call that fills them has been launched: after a failure the same input is
+    quantized again, by the layer itself and by the next one."""
+    to_q, to_k = Int8RotLinear(16, 16, group=16), Int8RotLinear(16, 16, group=16)
+    to_q.keep_input = True
+    x = torch.randn(4, 16).to(torch.bfloat16)
+    with monkeypatch.context() as m:
+        if fails == "status":
+            m.setattr(stub_library, "status", -4)
+        else:
+            empty = torch.empty
+
+            def refuse(*size, **kw):
+                if kw.get("dtype") is torch.bfloat16:
+                    raise torch.OutOfMemoryError("out of memory")
+                return empty(*size, **kw)
+
+            m.setattr(torch, "empty", refuse)
+        with pytest.raises(RuntimeError):
+            to_q._forward_one_call(x, x, (4,))
+    assert not Int8RotLinear._last_input
+    stub_library.quantized.clear()
+    to_k._forward_one_call(x, x, (4,))
+    to_q._forward_one_call(x, x, (4,))
+    to_k._forward_one_call(x, x, (4,))
+    assert stub_library.quantized == [False, False, True]
+    assert not Int8RotLinear._last_input
 
 
 def test_device_groups_are_checked():
