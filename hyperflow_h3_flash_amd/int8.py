@@ -124,9 +124,10 @@ class Int8RotLinear(nn.Module):
     rescaled by the token scale and the per-output-channel ``wscale``.
 
     Projections that share one input (q, k and v of an attention block) rotate and quantize it once: a layer whose
-    ``keep_input`` is set leaves ``(codes, scales)`` behind keyed by the input tensor's identity and version, the
-    next layer takes them when it is handed that very tensor unchanged, and every layer call drops what it did not
-    leave itself, so the codes never outlive the block (the cache of int8.py:150-159).
+    ``keep_input`` is set leaves ``(codes, scales)`` behind keyed by the input tensor's identity and version and the
+    stream they were computed on, the next layer takes them when it is handed that very tensor unchanged on that
+    stream, and every layer call drops what it did not leave itself, so the codes never outlive the block (the cache of
+    int8.py:150-159).
 
     ``rank``, ``bias`` and ``activation`` are this build's fused extension; with their defaults the module and its
     state dict are exactly the reference's. ``activation="gelu_tanh"`` applies torch's ``gelu(approximate="tanh")``
@@ -180,13 +181,17 @@ class Int8RotLinear(nn.Module):
         # Inference tensors (`torch.inference_mode`) have no version counter.
         version = None if x.is_inference() else x._version
         arithmetic = ARITHMETIC_OPTIONS["rotate_quant"]
+        # The codes are ordered (and their memory reused) on the stream that computes them: another stream's layer
+        # computes its own.
+        stream = _raw_stream(x2.get_device()) if x2.is_cuda else None
         entry = dict(cache)  # one copy: another thread may drop or replace the entry between the checks
         hit = (entry.get("x") is x and entry.get("version") == version and entry.get("group") == self.group
-               and entry.get("arithmetic") == arithmetic)
+               and entry.get("arithmetic") == arithmetic and entry.get("stream") == stream)
         quantized = entry["value"] if hit else kernels.rotate_quant(x2, self.group)
         cache.clear()
         if self.keep_input:
-            cache.update(x=x, version=version, group=self.group, arithmetic=arithmetic, value=quantized)
+            cache.update(x=x, version=version, group=self.group, arithmetic=arithmetic, stream=stream,
+                         value=quantized)
         return quantized
 
     def _forward_one_call(self, x: Tensor, x2: Tensor, shape: tuple[int, ...]) -> Tensor:
@@ -218,6 +223,7 @@ class Int8RotLinear(nn.Module):
                 _same_device(dev, t)
         cache = Int8RotLinear._last_input
         arithmetic = ARITHMETIC_OPTIONS["rotate_quant"]
+        stream = _raw_stream(index)
         keep, hit = self.keep_input, False
         xq = sx = None
         if cache or keep:
@@ -226,7 +232,7 @@ class Int8RotLinear(nn.Module):
             entry = dict(cache)
             version = None if x.is_inference() else x._version
             hit = (entry.get("x") is x and entry.get("version") == version and entry.get("group") == group
-                   and entry.get("arithmetic") == arithmetic)
+                   and entry.get("arithmetic") == arithmetic and entry.get("stream") == stream)
             if hit:
                 xq, sx = entry["value"]
             del entry
@@ -265,11 +271,11 @@ class Int8RotLinear(nn.Module):
             up.stride(0) if r else 0, r, None if bias is None else bias.data_ptr(), act, group,
             base + at_u if r else None, y.data_ptr(), n_out, M, N, K, base + at_ws if nbytes else None, nbytes)
         with _on(dev):
-            status = lib.hf_convrot_linear_ws(*args, _raw_stream(index))
+            status = lib.hf_convrot_linear_ws(*args, stream)
         _check(status, "hf_convrot_linear_ws")
         # Left behind only now: before the call xq and sx hold nothing, and a call that fails leaves nothing to share.
         if keep:
-            cache.update(x=x, version=version, group=group, arithmetic=arithmetic, value=(xq, sx))
+            cache.update(x=x, version=version, group=group, arithmetic=arithmetic, stream=stream, value=(xq, sx))
         return y
 
     def _forward_torch(self, x2: Tensor, rot: Tensor | None = None) -> Tensor:

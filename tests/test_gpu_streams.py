@@ -59,3 +59,46 @@ def test_concurrent_streams_match_serial_results():
     for j in (0, 1):
         for i, y in outs[j]:
             assert torch.equal(y, serial[i]), f"stream {j}, layer {i}"
+
+
+def test_layers_of_one_input_on_two_streams():
+    """A layer with keep_input on one stream and the next layer of the same input on another, neither waiting for the
+    other: each gives its serial bits, and the second leaves and takes no codes of the first's stream. The first stream
+    is kept busy, so that its codes come late; memory it freed is written over before the second is checked."""
+    from hyperflow_h3_flash_amd import Int8RotLinear
+
+    to_q, to_k = (_layer(1024, 2048, 32, False, seed=300 + i) for i in range(2))
+    x = torch.randn(512, 1024, generator=torch.Generator().manual_seed(9)).to(torch.bfloat16).to(DEV)
+    busy = torch.randn(4096, 4096, device=DEV)
+    print("stream test: shared input on two streams", flush=True)
+    with torch.no_grad():
+        want_q, want_k = to_q(x).clone(), to_k(x).clone()
+        torch.cuda.synchronize()
+        a, b = torch.cuda.Stream(DEV), torch.cuda.Stream(DEV)
+        for s in (a, b):
+            s.wait_stream(torch.cuda.current_stream(DEV))
+        to_q.keep_input = True
+        for _ in range(3):
+            with torch.cuda.stream(a):
+                for _ in range(3):
+                    late = busy @ busy
+                got_q = to_q(x)
+            assert Int8RotLinear._last_input["stream"] == a.cuda_stream
+            with torch.cuda.stream(b):
+                got_k = to_k(x)
+            assert not Int8RotLinear._last_input
+            with torch.cuda.stream(a):
+                over = torch.full((512, 1024), 3, device=DEV, dtype=torch.int8)
+            torch.cuda.synchronize()
+            assert torch.equal(got_q, want_q) and torch.equal(got_k, want_k)
+            del late, over
+        # on one stream they are still shared
+        with torch.cuda.stream(a):
+            got_q = to_q(x)
+            codes = Int8RotLinear._last_input["value"][0]
+            to_k.keep_input = True
+            got_k = to_k(x)
+            assert Int8RotLinear._last_input["value"][0] is codes
+        torch.cuda.synchronize()
+        assert torch.equal(got_q, want_q) and torch.equal(got_k, want_k)
+    Int8RotLinear._last_input.clear()

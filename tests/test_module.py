@@ -235,6 +235,38 @@ def test_a_failed_layer_leaves_no_codes_to_share(stub_library, monkeypatch, fail
     assert not Int8RotLinear._last_input
 
 
+def test_codes_are_shared_on_their_own_stream_only(stub_library, monkeypatch):
+    """The codes are ordered on the stream that computed them: a layer on another stream quantizes again, and what it
+    drops is not taken by a later layer either."""
+    current = [7]
+    monkeypatch.setattr(int8_mod, "_raw_stream", lambda index: current[0])
+    to_q, to_k, to_v = (Int8RotLinear(16, 16, group=16) for _ in range(3))
+    to_q.keep_input = to_k.keep_input = True
+    x = torch.randn(4, 16).to(torch.bfloat16)
+    for layer, stream in ((to_q, 7), (to_k, 8), (to_v, 7), (to_q, 7), (to_k, 7), (to_v, 7)):
+        current[0] = stream
+        layer._forward_one_call(x, x, (4,))
+    assert stub_library.quantized == [False, False, False, False, True, True]
+
+
+def test_composed_layers_share_codes_on_their_own_stream_only(monkeypatch):
+    """The same for the layer composed of separate kernel calls."""
+    current, calls = [7], []
+
+    class OnDevice(torch.Tensor):  # a host tensor that says it lies on a device
+        is_cuda = True
+
+    monkeypatch.setattr(int8_mod, "_raw_stream", lambda index: current[0])
+    kernels = SimpleNamespace(rotate_quant=lambda x2, group: calls.append(current[0]) or (x2, group))
+    to_q, to_k = Int8RotLinear(16, 16, group=16), Int8RotLinear(16, 16, group=16)
+    to_q.keep_input = True
+    x = torch.randn(4, 16).as_subclass(OnDevice)
+    for layer, stream in ((to_q, 7), (to_k, 8), (to_q, 8), (to_k, 8)):
+        current[0] = stream
+        layer._quantize(x, x, kernels)
+    assert calls == [7, 8, 8] and not Int8RotLinear._last_input
+
+
 def test_device_groups_are_checked():
     with pytest.raises(ValueError, match="power of 4"):
         int8_mod._check_group(128)
