@@ -66,10 +66,14 @@ SIGNATURES = {
                               _P, _P, _I64, _I64, _I64, _I64, _P, _I64, _P], ctypes.c_int),
     "hf_convrot_linear": ([_P, _I64, _P, _I64, _P, _P, _I64, _P, _I64, _I32, _P, _I32, _P, _P, _P, _P, _I64, _I64,
                            _I64, _I64, _P], ctypes.c_int),
+    "hf_route": ([_I32, _I64, _I64, _I64, _I32], ctypes.c_int32),
     "hf_convrot_linear_noalloc_max_bytes": ([], ctypes.c_int64),
     "hf_convrot_linear_noalloc": ([_P, _I64, _P, _P, _I32, _I32, _P, _I64, _P, _P, _I64, _P, _I64, _I32, _P, _I32,
                                    _I32, _P, _P, _I64, _I64, _I64, _I64, _P], ctypes.c_int),
 }
+
+#: Queries of hf_route.
+ROUTE_UP_ROWS = 0
 
 
 def hipcc() -> str:

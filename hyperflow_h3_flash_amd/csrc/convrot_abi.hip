@@ -691,6 +691,12 @@ bool use_up_tiles(int64_t M, int64_t N, int32_t r) {
   return r >= 128 && ((M + hf::GBM - 1) / hf::GBM) * ((N + hf::GBN - 1) / hf::GBN) >= device_cus();
 }
 
+// lowrank_up_rows_kernel's steps and workgroups (two per CU).
+int64_t up_rows_steps(int64_t M, int64_t N) {
+  return ((M + hf::kUrRows - 1) / hf::kUrRows) * ((N + hf::kUrCols - 1) / hf::kUrCols);
+}
+int64_t up_rows_grid(int64_t steps) { return std::min<int64_t>(2 * device_cus(), steps); }
+
 // Whether the up projection keeps u in registers and walks the columns (lowrank_up_rows_kernel): ranks up to 256 (the
 // registers), an output of whole 128-byte lines (its 64-column steps; with ragged lines M=6000, N=7000, r=136 took 64
 // against 55 us on the tiles), and enough (256 rows, 64 columns) steps that loading u and the first slab is a small
@@ -700,8 +706,18 @@ bool use_up_tiles(int64_t M, int64_t N, int32_t r) {
 // behind at 768 (M=1536, N=8192, r=192 10.8 -> 12.7), but up to rank 64 ahead from 512 steps on (M=2048, N=4096
 // 8.3 -> 6.9).
 bool use_up_rows(int64_t M, int64_t N, int32_t r) {
-  const int64_t steps = ((M + hf::kUrRows - 1) / hf::kUrRows) * ((N + hf::kUrCols - 1) / hf::kUrCols);
+  const int64_t steps = up_rows_steps(M, N);
   return r > 0 && r <= 256 && steps >= (r <= 64 ? 2 : 6) * (int64_t)device_cus() && steps < (int64_t(1) << 31);
+}
+
+// The multiplier that spreads lowrank_up_rows_kernel's workgroups over the columns, or 0. Where every share is the same
+// multiple of 8 steps and rows are whole KiB apart, all workgroups start at the same 128 bytes of a KiB and stay there
+// together: their stores meet in an eighth of the memory channels (M=65536, N=4096, 32 steps each: r=128 125 us on the
+// other kernels, 203 so, 124 from columns spread by a hash of the workgroup; r=192 148, 217, 122; M=32768, N=8192, r=64
+// 130, 197, 117). Other shares spread by themselves, and do better in their own order (M=101848, N=2048, r=128 99
+// against 115 us).
+uint32_t up_rows_turn(int64_t steps, int64_t grid, int64_t ldy) {
+  return ldy % 512 == 0 && steps % grid == 0 && steps / grid % 8 == 0 ? 0x9E3779B1u : 0u;
 }
 
 int64_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, int32_t r, int act_code) {
@@ -995,14 +1011,13 @@ int hf_lowrank_up(const uint16_t* u, int64_t ldu, const uint16_t* up, int64_t ld
   allow_large_lds();
   const int vec16 = aligned(y, 16) && (ldy % 8) == 0;
   if (!bias && aligned(y, 128) && (ldy % 64) == 0 && use_up_rows(M, N, r)) {
-    const int64_t steps_n = (N + hf::kUrCols - 1) / hf::kUrCols;
-    const int64_t steps = ((M + hf::kUrRows - 1) / hf::kUrRows) * steps_n;
-    const dim3 grid((unsigned)std::min<int64_t>(2 * device_cus(), steps)), block(hf::kUrThreads);
+    const int64_t steps = up_rows_steps(M, N), steps_n = (N + hf::kUrCols - 1) / hf::kUrCols;
+    const dim3 grid((unsigned)up_rows_grid(steps)), block(hf::kUrThreads);
     hipStream_t s = static_cast<hipStream_t>(stream);
 #define HF_UR_CASE(RC)                                                                                              \
   case RC:                                                                                                          \
     hipLaunchKernelGGL(hf::lowrank_up_rows_kernel<RC>, grid, block, hf::ur_lds(RC), s, u, ldu, up, ld_up, y, ldy,   \
-                       (int)M, (int)N, (int)r, (int)steps_n, (int)steps);                                           \
+                       (int)M, (int)N, (int)r, (int)steps_n, (int)steps, up_rows_turn(steps, grid.x, ldy));         \
     break;
     switch ((r + 63) / 64) { HF_UR_CASE(1) HF_UR_CASE(2) HF_UR_CASE(3) HF_UR_CASE(4) }
 #undef HF_UR_CASE
@@ -1200,6 +1215,18 @@ int hf_convrot_linear_ws(const uint16_t* x, int64_t ldx, int8_t* q, float* sx, i
   }
   return int8_linear_impl(q, K, w, ldw, sx, sw, u, r, up, ld_up, r, bias, y, ldy, M, N, K, ws, ws_bytes, stream,
                           activation);
+}
+
+int32_t hf_route(int32_t query, int64_t M, int64_t N, int64_t K, int32_t r) {
+  if (M <= 0 || N <= 0 || K < 0 || r < 0) return 0;
+  switch (query) {
+    case HF_ROUTE_UP_ROWS: {
+      if (!use_up_rows(M, N, r)) return 0;
+      const int64_t steps = up_rows_steps(M, N);
+      return up_rows_turn(steps, up_rows_grid(steps), N) ? 2 : 1;
+    }
+    default: return 0;
+  }
 }
 
 }  // extern "C"

@@ -766,7 +766,8 @@ __global__ __launch_bounds__(kUpThreads) void lowrank_up_kernel(const uint16_t* 
 // wave are waited for a step later, with the loads issued before them, and two workgroups share a CU, so one computes
 // while the other's stores drain; on the persistent 256 x 256 tiles a tile's stores had to drain before its second K
 // stage, with nothing else on the CU. A workgroup takes an equal share of all (256 rows, 64 columns) steps, columns
-// innermost, so the share may cross from one block of rows to the next. Sums in the order of the other up kernels (K
+// innermost, so the share may cross from one block of rows to the next; within a row block it may start in the middle of
+// its columns and go round (turn: the host's choice, up_rows_turn). Sums in the order of the other up kernels (K
 // ascending, 16 ranks per MFMA, up as the first operand): the same bits. Bound by the output's stores: M=37710,
 // N=7168 (541 MB written) takes 120-124 us at ranks 64 and 128, 4.4-4.5 TB/s where a plain fill reaches 4.5-4.9; 153
 // us at rank 256 (186 us on the tiles), whose 64 MFMAs per wave and step no longer hide behind them. u loaded in the
@@ -781,7 +782,8 @@ template <int RC>
 __global__ __launch_bounds__(kUrThreads, 2) void lowrank_up_rows_kernel(const uint16_t* __restrict__ u, int64_t ldu,
                                                                         const uint16_t* __restrict__ up, int64_t ldup,
                                                                         uint16_t* __restrict__ y, int64_t ldy, int M,
-                                                                        int N, int r, int steps_n, int steps) {
+                                                                        int N, int r, int steps_n, int steps,
+                                                                        uint32_t turn) {
   static_assert(2 * ur_lds(RC) <= 160 * 1024, "two workgroups per CU");
   extern __shared__ __attribute__((aligned(1024))) unsigned char ur_smem_raw[];
   unsigned char HF_LDS* smem = (unsigned char HF_LDS*)ur_smem_raw;
@@ -811,8 +813,13 @@ __global__ __launch_bounds__(kUrThreads, 2) void lowrank_up_rows_kernel(const ui
     }
   };
 
+  // The workgroup's columns [lo, hi) of row block mb, from step j on and round to it again (turn 0: from lo on).
+  int mb = first / steps_n, lo = first % steps_n, hi = min(steps_n, lo + last - first), left = hi - lo;
+  const uint32_t at = blockIdx.x * turn;
+  int j = lo + (int)__umulhi(at, (uint32_t)left);
+
   v8bf uf[4 * RC][2];
-  int mb = first / steps_n, j = first % steps_n, held = -1;
+  int held = -1;
   if (first < last) issue(j, smem);
   bool exact = false;  // the previous step issued exactly 8 stores per wave after its loads
   for (int t = first; t < last; ++t) {
@@ -856,7 +863,14 @@ __global__ __launch_bounds__(kUrThreads, 2) void lowrank_up_rows_kernel(const ui
         wave_lds_sync();
       }
     }
-    const int next_j = j + 1 < steps_n ? j + 1 : 0;
+    // The next step: on in this row block, or the share's columns of the next one.
+    int next_mb = mb, next_j = j + 1 < hi ? j + 1 : lo;
+    if (--left == 0) {
+      ++next_mb;
+      lo = 0;
+      left = hi = min(steps_n, last - t - 1);
+      next_j = (int)__umulhi(at, (uint32_t)left);
+    }
     if (t + 1 < last) issue(next_j, other);
 
     v16f acc[2][2];
@@ -955,17 +969,17 @@ __global__ __launch_bounds__(kUrThreads, 2) void lowrank_up_rows_kernel(const ui
     }
     exact = full;
     j = next_j;
-    if (next_j == 0) ++mb;
+    mb = next_mb;
   }
 }
 
 template __global__ void lowrank_up_rows_kernel<1>(const uint16_t*, int64_t, const uint16_t*, int64_t, uint16_t*,
-                                                   int64_t, int, int, int, int, int);
+                                                   int64_t, int, int, int, int, int, uint32_t);
 template __global__ void lowrank_up_rows_kernel<2>(const uint16_t*, int64_t, const uint16_t*, int64_t, uint16_t*,
-                                                   int64_t, int, int, int, int, int);
+                                                   int64_t, int, int, int, int, int, uint32_t);
 template __global__ void lowrank_up_rows_kernel<3>(const uint16_t*, int64_t, const uint16_t*, int64_t, uint16_t*,
-                                                   int64_t, int, int, int, int, int);
+                                                   int64_t, int, int, int, int, int, uint32_t);
 template __global__ void lowrank_up_rows_kernel<4>(const uint16_t*, int64_t, const uint16_t*, int64_t, uint16_t*,
-                                                   int64_t, int, int, int, int, int);
+                                                   int64_t, int, int, int, int, int, uint32_t);
 
 }  // namespace hf

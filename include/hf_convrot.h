@@ -198,6 +198,15 @@ int hf_convrot_linear_ws(const uint16_t* x, int64_t ldx, int8_t* q, float* sx, i
                          void* ws, int64_t ws_bytes, hf_stream_t stream);
 
 /*
+ * Which way a call of these sizes goes on the current device (256 CUs are assumed without one), for tests and
+ * measurements; nothing is launched, and every way gives the same bits. 0 for sizes or queries it does not know.
+ *   HF_ROUTE_UP_ROWS  hf_lowrank_up without a bias into dense rows of N (a multiple of 64, 128-byte aligned): 1 or 2 with
+ *                     u held in registers (2: its workgroups spread over the columns), 0 on tiles. K is not used.
+ */
+#define HF_ROUTE_UP_ROWS 0
+int32_t hf_route(int32_t query, int64_t M, int64_t N, int64_t K, int32_t r);
+
+/*
  * hf_convrot_linear_ws without the workspace argument, for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). No counterpart in the reference. It allocates
  * nothing: the split-K partial planes and low-rank partial sums live in a 64 MiB scratch array inside the library's

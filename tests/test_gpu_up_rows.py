@@ -28,14 +28,17 @@ def _device():
 
 # Steps of (256 rows, 64 columns), 512 workgroups: a share within one block of rows (N = 28672: 448 steps a block), and
 # shares that cross into the next; ragged last row blocks (one row, less and more than a wave's 64 rows of it); every
-# count of 64-rank chunks, full and with a partial last one; the fewest steps of the route (512 up to rank 64, else 1536).
-@pytest.mark.parametrize("m,n,r", [(2048, 4096, 8), (1793, 4096, 64), (8192, 4096, 72), (6017, 4096, 128),
-                                   (6200, 4096, 136), (24321, 1024, 192), (1000, 28672, 200), (12065, 2112, 256)])
-def test_up_rows_is_bitwise_the_other_kernels(oracle_lib, m, n, r):
+# count of 64-rank chunks, full and with a partial last one; the fewest steps of the route at several widths. Way 2 (equal
+# shares of a multiple of 8 steps): a share that is a part of a row block's columns, all of them, and several blocks.
+@pytest.mark.parametrize("m,n,r,way", [(2048, 4096, 8, 1), (1793, 4096, 64, 1), (8192, 4096, 72, 1),
+                                       (6017, 4096, 128, 1), (6200, 4096, 136, 1), (32513, 1024, 192, 1),
+                                       (1100, 28672, 200, 1), (27905, 2112, 256, 1), (50000, 192, 64, 1),
+                                       (32640, 2048, 200, 2), (131072, 512, 256, 2), (262100, 512, 64, 2)])
+def test_up_rows_is_bitwise_the_other_kernels(oracle_lib, m, n, r, way):
+    from hyperflow_h3_flash_amd import _native
     from hyperflow_h3_flash_amd.int8 import lowrank_up
 
-    steps = -(-m // 256) * -(-n // 64)
-    assert steps >= (512 if r <= 64 else 1536) and n % 64 == 0  # the route at 256 CUs
+    assert _native.library().hf_route(_native.ROUTE_UP_ROWS, m, n, 0, r) == way
     gen = torch.Generator(device=DEV).manual_seed(m + n + r)
     u = torch.randn(m, r, device=DEV, generator=gen).to(torch.bfloat16)
     up = (torch.randn(n, r, device=DEV, generator=gen) * 0.1).to(torch.bfloat16)
@@ -68,6 +71,7 @@ def test_up_rows_writes_only_its_columns(n):
     other = torch.full((m, ld + 8), 7.0, device=DEV, dtype=torch.bfloat16)
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     lib = _native.library()
+    assert lib.hf_route(_native.ROUTE_UP_ROWS, m, n, 0, r) == 1
     for out in (y, other):
         assert lib.hf_lowrank_up(u.data_ptr(), r, up.data_ptr(), r, r, None, out.data_ptr(), out.stride(0), m, n,
                                  stream) == 0
