@@ -699,15 +699,40 @@ int64_t up_rows_grid(int64_t steps) { return std::min<int64_t>(2 * device_cus(),
 
 // Whether the up projection keeps u in registers and walks the columns (lowrank_up_rows_kernel): ranks up to 256 (the
 // registers), an output of whole 128-byte lines (its 64-column steps; with ragged lines M=6000, N=7000, r=136 took 64
-// against 55 us on the tiles), and enough (256 rows, 64 columns) steps that loading u and the first slab is a small
-// part of a workgroup's share. Measured against the kernels it replaces there (us): M=37710, N=7168, r=256 186 -> 153,
-// r=192 172 -> 134, r=128 141 -> 124, r=96 159 -> 128, r=64 134 -> 120; N=28672, r=64 466 -> 435; M=41344, N=2048,
-// r=256 66 -> 55; M=8192, N=4096, r=256 (2048 steps) 42 -> 35; equal at 1504 steps (M=12000, N=2048, r=256 23.1) and
-// behind at 768 (M=1536, N=8192, r=192 10.8 -> 12.7), but up to rank 64 ahead from 512 steps on (M=2048, N=4096
-// 8.3 -> 6.9).
+// against 55 us on the tiles), and a rule by (256 rows, 64 columns) steps and by how well the other kernel's tiles
+// (128 columns below rank 128, 256 from there on) fit the width. Measured against the kernels it replaces over 5300
+// sizes, us before -> as these steps:
+//   * Up to rank 64 there is a band of sizes (10 to 48 steps per CU, past rank 48 15 to 40: outputs of about 80 to 400 MB
+//     on 256 CUs) where the tiles' ordinary stores still fit the Infinity Cache, and they stay ahead (M=32768, N=4096,
+//     r=16 50 -> 61, M=131072, N=1024, r=32 51 -> 60, M=8192, N=16384, r=64 54 -> 60), except where their columns are
+//     padding (N=192, r=32 33 -> 25) or, past rank 32, narrow (M=131072, N=512, r=64 34 -> 31). Fewer or more steps:
+//     M=16384, N=1024, r=32 12 -> 9; M=37710, N=7168, r=64 134 -> 120. N=128 only from 4 to 10 (M=131072, r=64 12.6 ->
+//     9.8; 24180 steps 204 -> 254).
+//   * Ranks 65 to 127: from 6 steps per CU on, ahead everywhere (M=37710, N=7168, r=96 159 -> 128).
+//   * From rank 128 on loading u is the larger part of a short share, and a share that crosses from one row block into
+//     the next loads it twice: at widths up to 1536 from 8 steps per CU (past rank 192 from 14) on, else from 6 on (6
+//     steps at M=24576, N=1024: r=256 23.8 -> 26.8; at N=512 24.3 -> 30.3; 16 steps at M=65536, N=1024, r=256 53 -> 46).
+//     N=256, one tile wide, only at rank 128 (M=196608, r=256 41.9 -> 45.3). Wide outputs: M=37710, N=7168, r=256 186 ->
+//     153, r=192 172 -> 134; M=8192, N=4096, r=256 42 -> 35.
 bool use_up_rows(int64_t M, int64_t N, int32_t r) {
-  const int64_t steps = up_rows_steps(M, N);
-  return r > 0 && r <= 256 && steps >= (r <= 64 ? 2 : 6) * (int64_t)device_cus() && steps < (int64_t(1) << 31);
+  if (r <= 0 || r > 256) return false;
+  const int64_t blocks = (M + hf::kUrRows - 1) / hf::kUrRows;
+  const int64_t steps = up_rows_steps(M, N), cus = device_cus();
+  if (steps >= (int64_t(1) << 31)) return false;
+  const int64_t tile = r < 128 ? hf::kUpTile : hf::GBN;
+  // Whether the other kernel's tiles fit the width (at most a tenth, or from rank 65 on a fifth, of them padding).
+  const bool fits = 10 * ((N + tile - 1) / tile * tile) < (r <= 64 ? 11 : 12) * N;
+  // The rows of the last block count in full here, in 128-row tiles there.
+  if (r < 128 && 4 * hf::kUrRows * blocks > 5 * hf::kUpTile * ((M + hf::kUpTile - 1) / hf::kUpTile)) return false;
+  if (r <= 64) {
+    if (fits && N <= 128) return steps >= 4 * cus && steps <= 10 * cus;
+    const bool behind = fits && (r <= 32 || N > 1024) && steps > (r > 48 ? 15 : 10) * cus &&
+                        steps < (r > 32 ? 40 : 48) * cus;
+    return steps >= 2 * cus && !behind;
+  }
+  if (r < 128 || !fits) return steps >= 6 * cus;
+  if (N <= 256) return r == 128 && steps >= 6 * cus && steps <= 32 * cus;
+  return steps >= (N > 1536 ? 6 : r <= 192 ? 8 : 14) * cus;
 }
 
 // The multiplier that spreads lowrank_up_rows_kernel's workgroups over the columns, or 0. Where every share is the same

@@ -18,6 +18,26 @@ def test_unknown_queries_and_sizes_are_zero():
     assert up(0, 4096, 64) == up(4096, 0, 64) == up(4096, 4096, 0) == up(37710, 7168, 264) == 0
 
 
+# Measured against the kernels it replaces (us, tiles -> u in registers): where it is behind it is not taken. Ranks up to
+# 64, outputs that the tiles leave in the Infinity Cache (50 -> 62, 51 -> 60, 23 -> 25, 38 -> 46, 54 -> 60); one tile of
+# 128 columns (204 -> 254); narrow outputs at large ranks (25 -> 31, 26 -> 32, 24 -> 27, 22 -> 25); few steps (10.8 ->
+# 12.7); 352 rows in blocks of 256.
+@pytest.mark.parametrize("m,n,r", [
+    (32768, 4096, 16), (131072, 1024, 32), (16384, 3072, 32), (14003, 7168, 16), (8192, 16384, 64), (3094835, 128, 64),
+    (49152, 512, 200), (98304, 256, 256), (24576, 1024, 256), (98304, 256, 136), (1536, 8192, 192), (352, 19072, 64),
+])
+def test_up_projection_stays_on_tiles_where_they_are_ahead(m, n, r):
+    assert up(m, n, r) == 0
+
+
+@pytest.mark.parametrize("m,n,r", [
+    (37710, 7168, 256), (37710, 7168, 64), (37710, 7168, 96), (41344, 2048, 256), (8192, 4096, 256),
+    (2048, 4096, 64), (16384, 1024, 32), (65536, 192, 32), (130000, 512, 64), (131072, 192, 256),
+])
+def test_up_projection_keeps_u_in_registers_where_that_is_ahead(m, n, r):
+    assert up(m, n, r) == 1
+
+
 # Equal shares of a multiple of 8 steps, rows whole KiB apart (us, tiles -> in step -> spread): 125 -> 203 -> 124,
 # 164 -> 217 -> 127, 130 -> 197 -> 117, 140 -> 171 -> 114.
 @pytest.mark.parametrize("m,n,r", [(65536, 4096, 128), (32768, 8192, 192), (32768, 8192, 64), (130995, 2048, 64)])
