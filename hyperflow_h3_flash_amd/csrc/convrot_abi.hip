@@ -421,11 +421,14 @@ int lowrank_down_impl(const uint16_t* x, int64_t ldx, const uint16_t* down, int6
     return HF_OK;
   }
   float* part = plan.splits > 1 ? static_cast<float*>(ws) : nullptr;
-  // A split projection runs before the layer's rotation, which reads x again. x that fits the eight XCDs' L2s (4 MiB
-  // each) is left there for it; a larger x is streamed past the caches: the rotation of that many rows is bound by its
-  // arithmetic, and x would push the codes and weights out. Layers, cached against streamed (same box, in turn): M=1000,
-  // K=5120 (10 MB) 50.1 against 50.7 us, M=1024, K=3072 30.2 against 31.0; M=5168, K=5120 (53 MB) 170.4 against 166.1,
-  // M=5168 feed-forward (53 and 143 MB) 813 against 811.
+  // Split launches leave an x of up to 32 MiB in the caches and stream a larger one past them. Its next reader is the
+  // layer's rotation (defer), the pass over the next 64 ranks, or the next layer of a shared input; where there is none
+  // (f32_recip, which rotates first; a low-rank linear alone) keeping it costs little. Kept against streamed, us: layers
+  // with the rotation next M=1024, K=N=3072, r=64 32.7 / 33.7, M=1000, K=5120 51.8 / 52.7, M=4096, K=1024 37.3 / 38.8,
+  // M=1000, K=13824 109.1 / 109.8; rank 128 M=2048, K=3072 80.1 / 81.6; f32_recip and shared codes within 1.3 %, shared
+  // codes M=1024, K=3072 28.0 / 28.9 where the call before read the same x; a low-rank linear alone on an x just written
+  // M=5400, K=3072, r=64 35.7 / 37.5, M=2048 25.2 / 25.7, but M=1000, K=5120 27.2 / 26.0. The line: the gain fades as x
+  // grows and is gone by 33 MB (M=3270, K=5120 125.0 / 124.7; 42 MB 155.6 / 156.4, 53 MB 169.3 / 169.0).
   const bool cache_x = part && 2 * M * K <= (int64_t(32) << 20);
   // Waves per workgroup (32 rows each): the fewest that cover the rows in one round of one workgroup per CU, from 4
   // (128 rows) to 8; split launches keep 4.

@@ -39,8 +39,8 @@ __device__ __forceinline__ int lr_swizzle(int row, int c) { return swizzle128(ro
 
 // One wave's share of a stage: `count` loads of 1 KiB (8 rows x 128 bytes) starting at LDS block `first_blk`.
 // Rows at or past `rows_valid`, and chunks at or past K, read as zero (offset `oob` is past the descriptor).
-// CPOL is the loads' cache policy: kCpolStream for x where this pass reads it last in a layer (after the rotation), so
-// its 2 bytes per element are not kept in the Infinity Cache over the codes the GEMM reads next.
+// CPOL is the loads' cache policy: kCpolStream for x where its 2 bytes per element are not to be kept in the Infinity
+// Cache over the codes the GEMM reads next (this pass reads it last, or it is large).
 constexpr int kCpolStream = 2;  // the nt (non-temporal) bit
 template <int COUNT, int CPOL = 0>
 __device__ __forceinline__ void lr_load(__amdgpu_buffer_rsrc_t rsrc, uint32_t oob, uint32_t ld_bytes, int rows_valid,
@@ -56,7 +56,7 @@ __device__ __forceinline__ void lr_load(__amdgpu_buffer_rsrc_t rsrc, uint32_t oo
   }
 }
 
-// CPOL: the cache policy of x's loads (the host's choice: 0 where the rotation reads a small x next).
+// CPOL: the cache policy of x's loads (the host's choice: 0 leaves a small x in the caches for its next reader).
 //
 // Split K (few rows): blockIdx.y = s covers K elements [s * k_chunk, (s + 1) * k_chunk) and writes its fp32 partial
 // sums to plane s of `part` ([splits][M][r]); lowrank_reduce_kernel, or in a layer the rotation kernel (LrFinish),
