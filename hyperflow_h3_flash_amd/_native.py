@@ -73,7 +73,7 @@ SIGNATURES = {
 }
 
 #: Queries of hf_route.
-ROUTE_UP_ROWS = 0
+ROUTE_UP_ROWS, ROUTE_ROTATE_LOWRANK, ROUTE_STREAM_WEIGHT = 0, 1, 2
 
 
 def hipcc() -> str:

@@ -748,6 +748,18 @@ uint32_t up_rows_turn(int64_t steps, int64_t grid, int64_t ldy) {
   return ldy % 512 == 0 && steps % grid == 0 && steps / grid % 8 == 0 ? 0x9E3779B1u : 0u;
 }
 
+// Whether mid_gemm_kernel streams the weight past the caches: one row of tiles (M <= 256) reads every weight panel
+// once, and a weight of more than half the 256 MiB Infinity Cache is gone from it before its next call if another of
+// that size is called in between, as in a model; it then only sweeps the codes out. Layers over four weights in turn,
+// kept against streamed (us): M=256, N=30720, K=5120 (150 MiB) 64.6 / 62.0, M=200 60.7 / 57.5, M=129 54.2 / 52.3; at
+// the line M=256, N=26368, K=5120 (129 MiB) 60.1 / 57.5, N=16640, K=8192 (130 MiB) 71.4 / 69.0; N=28672, K=8192 (224
+// MiB) 86.8 / 83.6. The price is one weight called alone over and over, which would stay: M=256
+// 57.5 / 61.4, 53.2 / 58.3, 64.6 / 69.4, 79.3 / 82.4; M=200, N=30720, K=5120 55.2 / 55.7. Smaller weights may still be
+// there from the call before (M=256, N=22016, K=3072, 64 MiB, called over three weights 35.9 / 39.1), and with more tile
+// rows the panels are read again (M=1024, N=7168, K=5120 57.9 / 59.8). The cache hints sc0 and sc1 instead cost nothing
+// with one weight, but gain half of it or less in turn (M=256, N=30720, K=5120 62.4, over whole calls 64.6 against 61.9).
+bool mid_streams_weight(int64_t M, int64_t N, int64_t K) { return M <= hf::kMidBM && N * K > (int64_t(128) << 20); }
+
 int64_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, int32_t r, int act_code) {
   if (M <= 0 || N <= 0 || K <= 0 || r < 0) return 0;
   return gemm_route(M, N, K, r, is_glu(act_code)).ws_bytes;
@@ -821,13 +833,7 @@ int int8_linear_impl(const int8_t* q, int64_t ldq, const int8_t* w, int64_t ldw,
     a.tiles_n = (int)((N + hf::kMidBN - 1) / hf::kMidBN);
     a.out_vec16 = aligned(y, 16) && (ldy % 8) == 0;
     const dim3 grid((unsigned)((int64_t)a.tiles_m * a.tiles_n)), block(hf::kMidThreads);
-    // One row of tiles (M <= 256) reads every weight panel once: a weight of more than half the 256 MiB Infinity Cache
-    // is streamed, so it leaves the codes in the L2s and does not sweep that cache for nothing. Layers, both orders on
-    // one box: M=256, N=30720, K=5120 (157 MB) 64.9 -> 62.8 us, M=200 62.0 -> 59.9, M=130, N=28672, K=5376 54.9 -> 54.0,
-    // K=7168 (220 MB) 79.5 -> 78.6. Smaller weights may still be there from the call before (M=256, N=22016, K=3072, 68
-    // MB, called over three weights 35.9 -> 39.1), and with more tile rows the panels are read again (M=1024, N=7168,
-    // K=5120 57.9 -> 59.8).
-    const bool stream_w = a.tiles_m == 1 && N * K > (int64_t(128) << 20);
+    const bool stream_w = mid_streams_weight(M, N, K);
 #define HF_MID_LAUNCH(ACT)                                                                                          \
     if (stream_w)                                                                                                   \
       hipLaunchKernelGGL((hf::mid_gemm_kernel<ACT, hf::kMidStreamW>), grid, block, hf::kMidLds, s, a);              \
@@ -1253,6 +1259,9 @@ int32_t hf_route(int32_t query, int64_t M, int64_t N, int64_t K, int32_t r) {
       const int64_t steps = up_rows_steps(M, N);
       return up_rows_turn(steps, up_rows_grid(steps), N) ? 2 : 1;
     }
+    case HF_ROUTE_ROTATE_LOWRANK: return r > 0 && rotate_lowrank_by_rows(M, K, r);
+    case HF_ROUTE_STREAM_WEIGHT:
+      return K > 0 && gemm_route(M, N, K, r, false).kind == GemmRoute::kMid && mid_streams_weight(M, N, K);
     default: return 0;
   }
 }

@@ -202,8 +202,13 @@ int hf_convrot_linear_ws(const uint16_t* x, int64_t ldx, int8_t* q, float* sx, i
  * measurements; nothing is launched, and every way gives the same bits. 0 for sizes or queries it does not know.
  *   HF_ROUTE_UP_ROWS  hf_lowrank_up without a bias into dense rows of N (a multiple of 64, 128-byte aligned): 1 or 2 with
  *                     u held in registers (2: its workgroups spread over the columns), 0 on tiles. K is not used.
+ *   HF_ROUTE_ROTATE_LOWRANK  hf_convrot_linear_ws (not quantized, HF_ROTATE_BF16_DIV, a group of at most 1024): 1 with
+ *                     the rotation and the low-rank down projection in one launch. N is not used.
+ *   HF_ROUTE_STREAM_WEIGHT  the INT8 GEMM without a gated activation: 1 with the weight streamed past the caches.
  */
 #define HF_ROUTE_UP_ROWS 0
+#define HF_ROUTE_ROTATE_LOWRANK 1
+#define HF_ROUTE_STREAM_WEIGHT 2
 int32_t hf_route(int32_t query, int64_t M, int64_t N, int64_t K, int32_t r);
 
 /*

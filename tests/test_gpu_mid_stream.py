@@ -24,9 +24,11 @@ def _device():
 @pytest.mark.parametrize("m,k,n,r,act", [(129, 5136, 30736, 0, None), (200, 5376, 28280, 24, "gelu_tanh"),
                                          (256, 5120, 30720, 64, None)])
 def test_streamed_weight_gives_the_bits_of_the_taller_product(m, k, n, r, act):
+    from hyperflow_h3_flash_amd import _native
     from hyperflow_h3_flash_amd.int8 import int8_matmul
 
-    assert n * k > 128 << 20 and -(-n // 128) <= 256 and 2 * -(-n // 128) > 256  # the route at 256 CUs
+    route = _native.library().hf_route
+    assert route(_native.ROUTE_STREAM_WEIGHT, m, n, k, r) == 1 and route(_native.ROUTE_STREAM_WEIGHT, 600, n, k, r) == 0
     gen = torch.Generator(device=DEV).manual_seed(m)
     rows = 600
     q = torch.randint(-127, 128, (rows, k), device=DEV, dtype=torch.int8, generator=gen)

@@ -23,13 +23,14 @@ def _device():
 
 # Both sides of the line: 3.5 rounds up to 5 tiles of 1024, 2 rounds past that (256 CUs holding 4 workgroups of 3 tiles,
 # 2 of 5 to 7); a partial last tile, a rank that is no multiple of 8 workgroup ranks, ranks past 64, another group.
-@pytest.mark.parametrize("m,k,r,group", [(384, 3072, 64, 256), (384, 3072, 72, 64), (384, 3072, 128, 256),
-                                         (298, 5120, 40, 256), (299, 5120, 40, 256), (193, 4864, 64, 256),
-                                         (204, 7168, 32, 1024), (205, 7168, 32, 1024), (193, 7168, 32, 16)])
-def test_row_launch_is_the_composed_layer(m, k, r, group):
-    from hyperflow_h3_flash_amd import Int8RotLinear
+@pytest.mark.parametrize("m,k,r,group,one", [(384, 3072, 64, 256, 1), (384, 3072, 72, 64, 0), (384, 3072, 128, 256, 0),
+                                             (298, 5120, 40, 256, 1), (299, 5120, 40, 256, 0), (193, 4864, 64, 256, 1),
+                                             (204, 7168, 32, 1024, 1), (205, 7168, 32, 1024, 0), (193, 7168, 32, 16, 1)])
+def test_row_launch_is_the_composed_layer(m, k, r, group, one):
+    from hyperflow_h3_flash_amd import Int8RotLinear, _native
     from hyperflow_h3_flash_amd.int8 import int8_matmul, lowrank_down, rotate_quant
 
+    assert _native.library().hf_route(_native.ROUTE_ROTATE_LOWRANK, m, 256, k, r) == one
     gen = torch.Generator(device=DEV).manual_seed(m + k + r)
     n = 256
     layer = Int8RotLinear(k, n, group, rank=r).to(DEV)

@@ -48,3 +48,27 @@ def test_up_projection_spreads_workgroups_that_would_store_in_step(m, n, r):
 @pytest.mark.parametrize("m,n,r", [(65536 + 256, 4096, 128), (65536, 4096 + 64, 128), (32768, 3072, 128)])
 def test_up_projection_leaves_other_shares_in_order(m, n, r):
     assert up(m, n, r) == 1
+
+
+def rotate_lowrank(m, k, r):
+    return _native.library().hf_route(_native.ROUTE_ROTATE_LOWRANK, m, 1, k, r)
+
+
+# Each side of each line: 128 rows, 192 at up to 7 tiles of 1024, then 3.5 rounds (up to 5 tiles) or 2 of the workgroups
+# that the CUs hold at once, while the projection alone would run by rows; up to 14 tiles.
+@pytest.mark.parametrize("m,k,r,one", [
+    (1, 3072, 64, 1), (128, 14336, 64, 1), (128, 14352, 64, 0), (129, 14336, 16, 0), (192, 7168, 64, 1),
+    (192, 8192, 64, 0), (193, 8192, 8, 1), (384, 3072, 64, 1), (384, 3072, 72, 0), (298, 5120, 40, 1), (299, 5120, 40, 0),
+    (204, 7168, 32, 1), (205, 7168, 32, 0), (332, 5120, 8, 1), (333, 5120, 8, 0), (385, 1024, 8, 0), (64, 5120, 0, 0),
+])
+def test_rotation_and_projection_in_one_launch(m, k, r, one):
+    assert rotate_lowrank(m, k, r) == one
+
+
+# One row of the 256 x 128 tiles and more than 128 MiB (26214.4 rows at K=5120), where those tiles run at all.
+@pytest.mark.parametrize("m,k,n,streamed", [
+    (256, 5120, 26216, 1), (256, 5120, 26208, 0), (257, 5120, 26216, 0), (129, 5120, 26216, 1), (128, 5120, 26216, 0),
+    (256, 8192, 16392, 1), (256, 8192, 16384, 0), (256, 5120, 32768, 1), (256, 5120, 32776, 0),
+])
+def test_streamed_weight(m, k, n, streamed):
+    assert _native.library().hf_route(_native.ROUTE_STREAM_WEIGHT, m, n, k, 32) == streamed
