@@ -114,6 +114,23 @@ def test_split_lowrank_down_matches_oracle(oracle_lib, m, k, r):
     assert (got == ref).mean() > 0.99
 
 
+# The partial sums go out four ranks at a time where the rank allows it, one by one where not: each side, in one 32-rank
+# block and in two, with a last group of four that is partly past the rank, and a second pass of 6 ranks.
+@pytest.mark.parametrize("r", [1, 4, 6, 28, 30, 33, 36, 60, 63, 70])
+def test_split_lowrank_down_of_any_rank_matches_oracle(oracle_lib, r):
+    from hyperflow_h3_flash_amd import _native
+    from hyperflow_h3_flash_amd.int8 import lowrank_down
+
+    m, k = 397, 5120
+    assert _native.library().hf_lowrank_down_ws_bytes(m, k, r) > 0, "this shape should take the split path"
+    inp = oracle_lib.make_inputs(m, k, 8, 256, rank=r, seed=r)
+    u = lowrank_down(to_dev_bf16(inp["x"]), to_dev_bf16(inp["down"]))
+    got = oracle_lib.bf16_to_f32(bits_of(u))
+    ref = oracle_lib.bf16_to_f32(oracle_lib.lowrank_down(inp["x"], inp["down"]))
+    assert within_fp32_sum_bound(got, ref, oracle_lib.bf16_to_f32(inp["x"]), oracle_lib.bf16_to_f32(inp["down"]))
+    assert (got == ref).mean() > 0.99
+
+
 @pytest.mark.parametrize("m,k,r", [(1, 5120, 32), (7, 1024, 8), (64, 5120, 64), (100, 13824, 32), (256, 5376, 32),
                                    (33, 16384, 136), (200, 3072, 40), (250, 7168, 64), (9, 2048, 12), (5, 1024, 1),
                                    (384, 5120, 32)])
