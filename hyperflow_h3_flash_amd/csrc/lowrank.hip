@@ -769,7 +769,7 @@ __global__ __launch_bounds__(kUpThreads) void lowrank_up_kernel(const uint16_t* 
 // innermost, so the share may cross from one block of rows to the next; within a row block it may start in the middle of
 // its columns and go round (turn: the host's choice, up_rows_turn). Sums in the order of the other up kernels (K
 // ascending, 16 ranks per MFMA, up as the first operand): the same bits. Bound by the output's stores: M=37710,
-// N=7168 (541 MB written) takes 120-124 us at ranks 64 and 128, 4.4-4.5 TB/s where a plain fill reaches 4.5-4.9; 153
+// N=7168 (541 MB written) takes 120-124 us at ranks 64 and 128, 4.4-4.5 TB/s where a plain fill reaches 4.6; 153
 // us at rank 256 (186 us on the tiles), whose 64 MFMAs per wave and step no longer hide behind them. u loaded in the
 // MFMA layout instead of whole lines cost 7 us at M=5168, N=5376.
 constexpr int kUrRows = 256, kUrCols = 64;
